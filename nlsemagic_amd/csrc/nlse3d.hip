@@ -14,6 +14,8 @@
 // Neighbour reads of the per-point kernels go through the L1/L2 caches: a
 // wavefront covers 64 consecutive k, so every plane and row neighbour is a
 // coalesced line read.
+#include <atomic>
+
 #include "nlse3d_cdpair.h"
 #include "nlse3d_march.h"
 #include "nlse3d_shocpair.h"
@@ -194,6 +196,54 @@ __global__ __launch_bounds__(NW * 64) void shocpair3d_kernel(const c2<T>* __rest
     shocpair_tile<T, FIRST, TJ, NW>(sm, ci * g.IC, jt * TJ, kt * 56, g, yin, u, acc, yout, V, c, BC, ulo);
 }
 
+// compute units of the current device
+static int device_cus()
+{
+    static std::atomic<int> cus{0};
+    int n = cus.load(std::memory_order_relaxed);
+    if (n == 0) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        cus.store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+// Planes per chunk of a pair launch with `cols` tiles per plane, H halo planes
+// per chunk and steps in groups of G.  A workgroup (one per CU) takes about
+// as long as its steps plus two for its first loads, so a launch takes
+// rounds(chunks) * (steps(chunk) + 2): short chunks fill the chip on small
+// grids, long ones spend less on halo planes.  Chunks of 32 planes stay where
+// nothing is 7 % better by this count (on grids of several rounds the count
+// is only good to a few per cent).
+// Time per step, chunks of 32 -> this rule: 64^3
+// CD FP64 79 -> 22 us, 2SHOC FP32 97 -> 31; 97 x 120 x 111 CD FP64 92 -> 47;
+// 192^3 CD FP64 223 -> 181, 2SHOC FP64 532 -> 462; 256^3 2SHOC FP64
+// 1087 -> 1014, CD FP64 476 -> 465.
+static int pair_chunk(int cols, int L, int H, int G)
+{
+    const int cus = device_cus();
+    auto cost = [&](int IC) -> long {
+        const long wgs = (long)cols * ((L + IC - 1) / IC);
+        return (wgs + cus - 1) / cus * ((IC + H + G - 1) / G * G + 2);
+    };
+    const int base = 32;
+    int best = base;
+    long bc = cost(base) * 93;  // hundredths
+    for (int n = 1; n <= (L + 3) / 4; ++n) {
+        const int IC = (L + n - 1) / n;
+        if (IC < 4 || IC > 96) continue;
+        const long k = cost(IC) * 100;
+        if (k < bc) {
+            bc = k;
+            best = IC;
+        }
+    }
+    return best;
+}
+
 template <typename T>
 static hipError_t launch_shocpair3d(const StageArgs<T>& a, bool first, hipStream_t st)
 {
@@ -205,9 +255,9 @@ static hipError_t launch_shocpair3d(const StageArgs<T>& a, bool first, hipStream
     g.N = a.N;
     g.M = a.M;
     g.L = a.L;
-    g.IC = 32;
     g.tj = (a.N + TJ - 1) / TJ;
     g.tk = (a.M + 55) / 56;
+    g.IC = pair_chunk(g.tj * g.tk, a.L, 8, 4);
     g.ti = (a.L + g.IC - 1) / g.IC;
     g.per_xcd = (g.tj * g.tk * g.ti + 7) / 8;
     if (first)
@@ -233,9 +283,9 @@ hipError_t launch_pair3d(const StageArgs<T>& a, bool first, hipStream_t st)
     g.N = a.N;
     g.M = a.M;
     g.L = a.L;
-    g.IC = 32;
     g.tj = (a.N + TJ - 1) / TJ;
     g.tk = (a.M + 59) / 60;
+    g.IC = pair_chunk(g.tj * g.tk, a.L, 4, 3);
     g.ti = (a.L + g.IC - 1) / g.IC;
     g.per_xcd = (g.tj * g.tk * g.ti + 7) / 8;
     if (first)

@@ -1,0 +1,48 @@
+"""Tiling of the 3D two-stage launches: chunk lengths chosen by grid size.
+
+The chunk length along the first axis depends on the number of tiles per
+plane, so grids are picked whose last chunk, row tile or column tile holds one
+point, or whose chunks are the shortest and longest the rule gives.  Results
+must not depend on the tiling: they equal one stage per launch bit for bit.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import nlsemagic_amd as nm
+    if nm.device_count() < 1:
+        pytest.fail("no HIP device visible")
+    return nm
+
+
+def _run(hip, shape, method, prec, BC, fusion, U, V, steps):
+    sol = hip.Solver(shape, method, prec, BC, -1.0, 0.9, 0.04, 0.004)
+    sol.set_fusion(fusion)
+    sol.set_state(U, V)
+    sol.step(steps)
+    got = sol.state()
+    sol.close()
+    return got
+
+
+def _field(shape, seed):
+    rng = np.random.default_rng(seed)
+    U = (0.9 + 0.3 * rng.uniform(-1, 1, shape)) + 1j * (0.3 * rng.uniform(-1, 1, shape))
+    return U, 0.5 * rng.uniform(-1, 1, shape)
+
+
+@pytest.mark.parametrize("prec", [2, 1, 3])
+@pytest.mark.parametrize("method", [1, 2])
+@pytest.mark.parametrize("shape,BC", [((41, 25, 121), 1), ((13, 300, 57), 3), ((200, 100, 61), 1), ((7, 5, 113), 3)])
+def test_pair3d_chunk_lengths(hip, shape, BC, method, prec):
+    print("CASE", shape, BC, method, prec, flush=True)
+    U, V = _field(shape, sum(shape) + method)
+    assert bits_equal(_run(hip, shape, method, prec, BC, 2, U, V, 3), _run(hip, shape, method, prec, BC, 1, U, V, 3))
