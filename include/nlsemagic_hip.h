@@ -249,9 +249,10 @@ int nlse_vortex_profile(int m, double OM, double a, double s, double hr, int n, 
 int nlse_profile_launches(nlse_solver *h, int steps, double *ms_launch, int *nlaunch);
 /* RK4 stages fused per kernel launch (the results are identical for every
  * choice): 2D 1, 2 or 4 (default 4, a whole step per launch); 3D 1 or 2
- * (default 2: two stages per plane-marching launch, CD and 2SHOC, with a
- * boundary other than MSD and planes of fewer than 2^31 points; MSD runs one
- * stage per launch) */
+ * (default 2: two stages per plane-marching launch, CD and 2SHOC, planes of
+ * fewer than 2^31 points; MSD grids of fewer than 400,000 points, double
+ * 2SHOC ones of fewer than 2,500,000, run one stage per launch, which is
+ * faster there) */
 int nlse_set_fusion(nlse_solver *h, int stages_per_launch);
 /* 2D: the stage kernel family and its rows per tile (results identical for
  * every choice):
@@ -262,9 +263,9 @@ int nlse_set_fusion(nlse_solver *h, int stages_per_launch);
  *           of 3..256 rows, for 1, 2 or 4 stages per launch
  * 3D 2SHOC, one stage per launch: kind 1 (default) marches planes with D
  * kept on chip, tiles of 4 (default) or 8 rows x 60 columns; kind 0 runs a D
- * pass and an F pass per stage.  MSD boundaries always use the two passes.
- * Two stages per launch (nlse_set_fusion) march tiles of 4 rows x 56
- * columns (2SHOC) or 4 x 60 (CD) whatever the kind.
+ * pass and an F pass per stage; MSD boundaries use the two passes there.
+ * Two stages per launch (nlse_set_fusion) march tiles of 4, 8 or 12 rows x 56
+ * columns (2SHOC) or 12 x 60 (CD) whatever the kind.
  * 1D: kind 1 (default) advances `rows` steps (1..80 CD, 1..32 2SHOC; default
  * 32 CD, 16 2SHOC) per launch on windows of 64-256 points with a halo, one per CU;
  * kind 0 runs a whole chunk in one workgroup (N <= 4096) or one launch per

@@ -4,6 +4,9 @@
 // (:28-223) and NLSE3D_TAKE_STEPS_2SHOC.c (:28-412), with the chunk loop of
 // :308-322 / :507-521 on the host.  Element (i, j, k) is at (i*N + j)*M + k:
 // i < L slowest, k < M contiguous.
+// By default two stages per launch on plane-marching tiles (nlse3d_cdpair.h,
+// nlse3d_shocpair.h).  One stage per launch (on request, and on small MSD
+// grids):
 //   CD:    one fused kernel per RK4 stage (7-point stencil + BC + update).
 //   2SHOC: one plane-marching kernel per RK4 stage that keeps D on chip
 //          (nlse3d_march.h); for MSD boundaries, whose partner can lie in
@@ -156,6 +159,7 @@ static hipError_t launch_march3d(const StageArgs<T>& a, int IC, hipStream_t st)
     g.M = a.M;
     g.L = a.L;
     g.IC = IC;
+    g.ioff = g.joff = g.koff = 0;
     g.tj = (a.N + TJ - 1) / TJ;
     g.tk = (a.M + March3Cfg<TJ>::W - 1) / March3Cfg<TJ>::W;
     g.ti = (a.L + IC - 1) / IC;
@@ -165,35 +169,52 @@ static hipError_t launch_march3d(const StageArgs<T>& a, int IC, hipStream_t st)
     return hipGetLastError();
 }
 
+// whether the extended tile (owned points plus H on each side) of a pair
+// launch reaches the grid's boundary
+template <int TJ, int W, int H>
+__device__ __forceinline__ bool pair_edge(const March3& g, int i0, int j0, int k0)
+{
+    return i0 - H <= 0 || i0 + g.IC + H >= g.L || j0 - H <= 0 || j0 + TJ + H >= g.N || k0 - H <= 0 ||
+           k0 + W + H >= g.M;
+}
+
 // CD, two stages per launch (stages 1-2 or 3-4) on plane-marching tiles
-template <typename T, int FIRST, int TJ, int NW>
+template <typename T, int FIRST, int TJ, int NW, bool MSD>
 __global__ __launch_bounds__(NW * 64) void cdpair3d_kernel(const c2<T>* __restrict__ yin, const c2<T>* u,
                                                            c2<T>* __restrict__ acc, c2<T>* __restrict__ yout,
                                                            const T* __restrict__ V, Coefs<T> c, March3 g, int BC,
                                                            c2<T>* ulo)
 {
-    __shared__ CdPairLds<T, TJ> sm;
+    __shared__ CdPairLds<T, TJ, MSD> sm;
     const int t = (blockIdx.x & 7) * g.per_xcd + (blockIdx.x >> 3);
     if (t >= g.tj * g.tk * g.ti) return;
     const int kt = t % g.tk, rest = t / g.tk;
     const int jt = rest % g.tj, ci = rest / g.tj;
-    cdpair_tile<T, FIRST, TJ, NW>(sm, ci * g.IC, jt * TJ, kt * 60, g, yin, u, acc, yout, V, c, BC, ulo);
+    const int i0 = ci * g.IC - g.ioff, j0 = jt * TJ - g.joff, k0 = kt * 60 - g.koff;
+    if (MSD && pair_edge<TJ, 60, 2>(g, i0, j0, k0))
+        cdpair_tile<T, FIRST, TJ, NW, MSD>(sm, i0, j0, k0, g, yin, u, acc, yout, V, c, BC, ulo);
+    else
+        cdpair_tile<T, FIRST, TJ, NW, false>(sm, i0, j0, k0, g, yin, u, acc, yout, V, c, BC, ulo);
 }
 
-// 2SHOC, two stages per launch on plane-marching tiles (one extended row per
-// wave; D and the running ktot in LDS)
-template <typename T, int FIRST, int TJ, int NW>
-__global__ __launch_bounds__(NW * 64) void shocpair3d_kernel(const c2<T>* __restrict__ yin, const c2<T>* u,
-                                                             c2<T>* __restrict__ acc, c2<T>* __restrict__ yout,
-                                                             const T* __restrict__ V, Coefs<T> c, March3 g, int BC,
-                                                             c2<T>* ulo)
+// 2SHOC, two stages per launch on plane-marching tiles
+template <typename T, int FIRST, int TJ, bool MSD>
+__global__ __launch_bounds__((TJ + 4) * 64) void shocpair3d_kernel(const c2<T>* __restrict__ yin, const c2<T>* u,
+                                                                   c2<T>* __restrict__ acc, c2<T>* __restrict__ yout,
+                                                                   const T* __restrict__ V, Coefs<T> c, March3 g,
+                                                                   int BC, c2<T>* ulo)
 {
-    __shared__ ShocPairLds<T, TJ> sm;
+    using Lds = ShocPairLds<T, TJ, MSD>;
+    __shared__ Lds sm;
     const int t = (blockIdx.x & 7) * g.per_xcd + (blockIdx.x >> 3);
     if (t >= g.tj * g.tk * g.ti) return;
     const int kt = t % g.tk, rest = t / g.tk;
     const int jt = rest % g.tj, ci = rest / g.tj;
-    shocpair_tile<T, FIRST, TJ, NW>(sm, ci * g.IC, jt * TJ, kt * 56, g, yin, u, acc, yout, V, c, BC, ulo);
+    const int i0 = ci * g.IC - g.ioff, j0 = jt * TJ - g.joff, k0 = kt * 56 - g.koff;
+    if (MSD && pair_edge<TJ, 56, 4>(g, i0, j0, k0))
+        ShocPair<T, FIRST, TJ, MSD, Lds>(sm, i0, j0, k0, g, yin, u, acc, yout, V, c, BC, ulo).run();
+    else
+        ShocPair<T, FIRST, TJ, false, Lds>(sm, i0, j0, k0, g, yin, u, acc, yout, V, c, BC, ulo).run();
 }
 
 // compute units of the current device
@@ -217,11 +238,10 @@ static int device_cus()
 // rounds(chunks) * (steps(chunk) + 2): short chunks fill the chip on small
 // grids, long ones spend less on halo planes.  Chunks of 32 planes stay where
 // nothing is 7 % better by this count (on grids of several rounds the count
-// is only good to a few per cent).
-// Time per step, chunks of 32 -> this rule: 64^3
-// CD FP64 79 -> 22 us, 2SHOC FP32 97 -> 31; 97 x 120 x 111 CD FP64 92 -> 47;
-// 192^3 CD FP64 223 -> 181, 2SHOC FP64 532 -> 462; 256^3 2SHOC FP64
-// 1087 -> 1014, CD FP64 476 -> 465.
+// is only good to a few per cent).  Time per step, chunks of 32 -> this rule:
+// 64^3 CD FP64 79 -> 22 us, 2SHOC FP64 112 -> 33; 97 x 120 x 111 CD FP64
+// 92 -> 47, 2SHOC FP64 121 -> 70; 192^3 CD FP64 223 -> 181, 2SHOC FP64
+// 373 -> 317; 256^3 unchanged within 2 %.
 static int pair_chunk(int cols, int L, int H, int G)
 {
     const int cus = device_cus();
@@ -244,57 +264,64 @@ static int pair_chunk(int cols, int L, int H, int G)
     return best;
 }
 
-template <typename T>
-static hipError_t launch_shocpair3d(const StageArgs<T>& a, bool first, hipStream_t st)
+// the tiles of a pair launch: TJ rows x W columns over chunks of planes (a
+// halo of H on each side); MSD tiles own at least two points of the grid
+// along every axis
+static March3 pair_tiles(int N, int M, int L, int TJ, int W, int H, int G, bool msd)
 {
-    // FP64: 4 owned rows on 12 waves (LDS rings of 160 KiB, one workgroup
-    // per CU); FP32: 8 rows on 16 waves (120 KiB)
-    constexpr int TJ = std::is_same<T, double>::value ? 4 : 8, NW = TJ + 8;
-    if ((long)a.N * a.M > 0x7fffffffL) return hipErrorInvalidValue;  // 32-bit offsets within a plane
     March3 g;
-    g.N = a.N;
-    g.M = a.M;
-    g.L = a.L;
-    g.tj = (a.N + TJ - 1) / TJ;
-    g.tk = (a.M + 55) / 56;
-    g.IC = pair_chunk(g.tj * g.tk, a.L, 8, 4);
-    g.ti = (a.L + g.IC - 1) / g.IC;
+    g.N = N;
+    g.M = M;
+    g.L = L;
+    g.joff = msd && N % TJ == 1;
+    g.koff = msd && M % W == 1;
+    g.tj = (N + g.joff + TJ - 1) / TJ;
+    g.tk = (M + g.koff + W - 1) / W;
+    g.IC = pair_chunk(g.tj * g.tk, L, 2 * H, G);
+    g.ioff = msd && L % g.IC == 1;
+    g.ti = (L + g.ioff + g.IC - 1) / g.IC;
     g.per_xcd = (g.tj * g.tk * g.ti + 7) / 8;
-    if (first)
-        hipLaunchKernelGGL((shocpair3d_kernel<T, 1, TJ, NW>), dim3(8 * g.per_xcd), dim3(NW * 64), 0, st, a.yin, a.u,
-                           a.acc, a.yout, a.V, a.c, g, a.BC, a.ulo);
-    else
-        hipLaunchKernelGGL((shocpair3d_kernel<T, 3, TJ, NW>), dim3(8 * g.per_xcd), dim3(NW * 64), 0, st, a.yin, a.u,
-                           a.acc, a.yout, a.V, a.c, g, a.BC, a.ulo);
+    return g;
+}
+
+template <typename T, int FIRST, bool MSD>
+static hipError_t launch_shocpair3d(const StageArgs<T>& a, hipStream_t st)
+{
+    // the most rows whose register rings fit: TJ + 4 waves of 168 (12 waves),
+    // 128 (16) or, for double MSD, 209 VGPRs (8)
+    constexpr int TJ = std::is_same<T, double>::value ? (MSD ? 4 : 8) : 12;
+    if ((long)a.N * a.M > 0x7fffffffL) return hipErrorInvalidValue;  // 32-bit offsets within a plane
+    const March3 g = pair_tiles(a.N, a.M, a.L, TJ, 56, 4, 4, MSD);
+    hipLaunchKernelGGL((shocpair3d_kernel<T, FIRST, TJ, MSD>), dim3(8 * g.per_xcd), dim3((TJ + 4) * 64), 0, st, a.yin,
+                       a.u, a.acc, a.yout, a.V, a.c, g, a.BC, a.ulo);
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_pair3d(const StageArgs<T>& a, bool first, hipStream_t st)
+template <typename T, int FIRST, bool MSD>
+static hipError_t launch_cdpair3d(const StageArgs<T>& a, hipStream_t st)
 {
-    if (a.method == 2) return launch_shocpair3d<T>(a, first, st);
     // 12 owned rows on 16 waves, one extended row per wave: few registers
     // per wave (stages 3-4 in FP64: 117 VGPRs, against 208 with two rows per
     // wave) and j-halo rows re-read through L2 for 12 owned rows instead of
     // 4 (the halo re-reads dominate the HBM traffic beyond the 128 B per
     // point-step the pair needs)
     constexpr int TJ = 12, NW = TJ + 4;
-    March3 g;
-    g.N = a.N;
-    g.M = a.M;
-    g.L = a.L;
-    g.tj = (a.N + TJ - 1) / TJ;
-    g.tk = (a.M + 59) / 60;
-    g.IC = pair_chunk(g.tj * g.tk, a.L, 4, 3);
-    g.ti = (a.L + g.IC - 1) / g.IC;
-    g.per_xcd = (g.tj * g.tk * g.ti + 7) / 8;
-    if (first)
-        hipLaunchKernelGGL((cdpair3d_kernel<T, 1, TJ, NW>), dim3(8 * g.per_xcd), dim3(NW * 64), 0, st, a.yin, a.u,
-                           a.acc, a.yout, a.V, a.c, g, a.BC, a.ulo);
-    else
-        hipLaunchKernelGGL((cdpair3d_kernel<T, 3, TJ, NW>), dim3(8 * g.per_xcd), dim3(NW * 64), 0, st, a.yin, a.u,
-                           a.acc, a.yout, a.V, a.c, g, a.BC, a.ulo);
+    const March3 g = pair_tiles(a.N, a.M, a.L, TJ, 60, 2, 3, MSD);
+    hipLaunchKernelGGL((cdpair3d_kernel<T, FIRST, TJ, NW, MSD>), dim3(8 * g.per_xcd), dim3(NW * 64), 0, st, a.yin,
+                       a.u, a.acc, a.yout, a.V, a.c, g, a.BC, a.ulo);
     return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_pair3d(const StageArgs<T>& a, bool first, hipStream_t st)
+{
+    const bool msd = a.BC == BC_MSD;
+    if (a.method == 2) {
+        if (msd) return first ? launch_shocpair3d<T, 1, true>(a, st) : launch_shocpair3d<T, 3, true>(a, st);
+        return first ? launch_shocpair3d<T, 1, false>(a, st) : launch_shocpair3d<T, 3, false>(a, st);
+    }
+    if (msd) return first ? launch_cdpair3d<T, 1, true>(a, st) : launch_cdpair3d<T, 3, true>(a, st);
+    return first ? launch_cdpair3d<T, 1, false>(a, st) : launch_cdpair3d<T, 3, false>(a, st);
 }
 
 template hipError_t launch_pair3d<double>(const StageArgs<double>&, bool, hipStream_t);

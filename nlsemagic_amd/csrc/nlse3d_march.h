@@ -33,6 +33,9 @@ struct March3 {
     int IC;          // planes per chunk
     int tj, tk, ti;  // tiles along j, k and chunks along i
     int per_xcd;     // workgroups per XCD
+    // the first tile of each axis starts at -off (0, or 1 where the last one
+    // would own a single point and the boundary rule needs its neighbour too)
+    int ioff, joff, koff;
 };
 
 template <int TJ, int NW = 4>

@@ -319,13 +319,23 @@ void drop_graphs(nlse_solver* h)
     }
 }
 
-// RK4 stages per launch actually used: 2D 1, 2 or 4; 3D pairs of stages
-// (not MSD, whose partner may lie in another plane, nor planes of 2^31 points
-// or more, beyond the pair kernels' 32-bit offsets); 1 otherwise
+// 3D MSD: whether two stages per launch beat one.  Tiles at the boundary take
+// a second barrier and a division per stencil, and small grids are all
+// boundary.  Per step, one stage / two: CD FP64 64^3 22 / 28 us, 80^3 45 / 29;
+// 2SHOC FP32c 64^3 48 / 55, 80^3 107 / 76; 2SHOC FP64 (4-row tiles) 64^3 54 /
+// 67, 97 x 120 x 111 203 / 173, 128^3 261 / 307, 157 x 149 x 163 642 / 371.
+bool msd_pairs(const nlse_solver* h)
+{
+    return h->n >= (h->method == 2 && h->prec == 2 ? 2500000 : 400000);
+}
+
+// RK4 stages per launch actually used: 2D 1, 2 or 4; 3D pairs of stages (MSD
+// from a size on; not planes of 2^31 points or more, beyond the pair kernels'
+// 32-bit offsets); 1 otherwise
 int fusion(const nlse_solver* h)
 {
     if (h->dim == 2) return h->fuse;
-    if (h->dim == 3 && h->BC != BC_MSD && h->fuse == 2 && (long)h->N * h->M <= 0x7fffffffL) return 2;
+    if (h->dim == 3 && h->fuse == 2 && (long)h->N * h->M <= 0x7fffffffL && (h->BC != BC_MSD || msd_pairs(h))) return 2;
     return 1;
 }
 

@@ -139,6 +139,22 @@ template <typename T> __device__ __forceinline__ c2<T> msd_f(c2<T> fq, c2<T> uq,
     return mk<T>(-om * ub.y, om * ub.x);
 }
 
+// the same in two parts: the partner's rate om = Im(F/U), and F of a boundary
+// point from it (one om serves every boundary point of that partner)
+template <typename T> __device__ __forceinline__ T msd_rate(c2<T> fq, c2<T> uq)
+{
+    return (fq.y * uq.x - fq.x * uq.y) / (uq.x * uq.x + uq.y * uq.y);
+}
+template <typename T> __device__ __forceinline__ c2<T> msd_om(T om, c2<T> ub) { return mk<T>(-om * ub.y, om * ub.x); }
+
+// lane = column k of a row of M columns: the value of the column's MSD
+// partner (columns 0 and M-1 take their inward neighbour's, others their own)
+template <typename T> __device__ __forceinline__ T msd_col(T v, int k, int M)
+{
+    const T p = lane_shift<DPP_NEXT>(v), m = lane_shift<DPP_PREV>(v);
+    return k == 0 ? p : (k == M - 1 ? m : v);
+}
+
 // MSD: boundary D from the partner's D (NLSEmagic2D_CPU.c:297-303)
 template <typename T>
 __device__ __forceinline__ c2<T> msd_d(c2<T> dq, c2<T> uq, T vq, c2<T> ub, T vb, const Coefs<T>& c)

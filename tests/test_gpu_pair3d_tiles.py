@@ -46,3 +46,34 @@ def test_pair3d_chunk_lengths(hip, shape, BC, method, prec):
     print("CASE", shape, BC, method, prec, flush=True)
     U, V = _field(shape, sum(shape) + method)
     assert bits_equal(_run(hip, shape, method, prec, BC, 2, U, V, 3), _run(hip, shape, method, prec, BC, 1, U, V, 3))
+
+
+def _msd_cases():
+    """MSD pairs: thin grids along each axis, last tiles of one row, column
+    or plane (the tiles then shift by one), several tiles per axis; double
+    2SHOC runs pairs on larger grids only."""
+    small = [(3, 400, 400), (401, 3, 400), (400, 401, 3), (65, 97, 121), (97, 61, 113), (41, 97, 169), (81, 85, 61)]
+    large = [(3, 1001, 900), (1001, 3, 900), (900, 1001, 3), (129, 137, 169), (98, 229, 113)]
+    return [(sh, m, pr) for m in (1, 2) for pr in (2, 1, 3) for sh in (large if (m, pr) == (2, 2) else small)]
+
+
+@pytest.mark.parametrize("shape,method,prec", _msd_cases())
+def test_pair3d_msd_matches_one_stage(hip, shape, method, prec):
+    """Two MSD stages per launch give the bits of one stage per launch, NaN
+    and infinities included where a partner point is zero."""
+    print("CASE", shape, method, prec, flush=True)
+    U, V = _field(shape, sum(shape) + method)
+    sol = hip.Solver(shape, method, prec, 2, -1.0, 0.9, 0.04, 0.004)
+    assert sol.config()[0] == 2
+    sol.close()
+    assert bits_equal(_run(hip, shape, method, prec, 2, 2, U, V, 3), _run(hip, shape, method, prec, 2, 1, U, V, 3))
+    U[1, 1, 1] = U[-2, shape[1] // 2, -2] = U[shape[0] // 2, -2, shape[2] // 2] = 0
+    a = _run(hip, shape, method, prec, 2, 2, U, V, 1)
+    assert bits_equal(a, _run(hip, shape, method, prec, 2, 1, U, V, 1)) and np.isnan(a.real).any()
+
+
+@pytest.mark.parametrize("shape,method", [((65, 97, 121), 1), ((98, 229, 113), 2)])
+def test_pair3d_msd_matches_oracle(hip, oracle, shape, method):
+    U, V = _field(shape, sum(shape))
+    exp = oracle.take_steps(U, V, -1.0, 0.9, 0.04, 2, 2, 0.004, method)
+    assert bits_equal(_run(hip, shape, method, 2, 2, 2, U, V, 2), exp)
