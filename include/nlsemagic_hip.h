@@ -89,6 +89,12 @@ int NLSE3D_TAKE_STEPS_HIP_F(const float *Uoldr, const float *Uoldi, const float 
 int NLSE3D_VORTICITY_HIP(const double *Ur, const double *Ui, double lh2, double veps, int M, int N, int L,
                          double *wx, double *wy, double *wz, double *W);
 
+/* NLSE{1,2,3}D_TAKE_STEPS_HIP (precision 2) or _HIP_F (precision 1: U, V and the
+ * scalars rounded to float, the result widened) on interleaved complex arrays
+ * of doubles; unused sizes are passed as 1 */
+int nlse_take_steps_z(int dim, const double *U, const double *V, double *Unew, double s, double a, double h2, int BC,
+                      int chunk_size, double k, int N, int M, int L, int method, int precision);
+
 /* ---- resident-state API ---- */
 typedef struct nlse_solver nlse_solver;
 
@@ -106,6 +112,11 @@ int nlse_set_state_f(nlse_solver *h, const float *Ur, const float *Ui, const flo
 /* device state -> host planes (synchronises the solver's stream) */
 int nlse_get_state(nlse_solver *h, double *Ur, double *Ui);
 int nlse_get_state_f(nlse_solver *h, float *Ur, float *Ui);
+/* the same with interleaved complex arrays of doubles (re, im per point, C's
+ * double _Complex or numpy's complex128), which double states take without a
+ * conversion; V may be NULL */
+int nlse_set_state_z(nlse_solver *h, const double *U, const double *V);
+int nlse_get_state_z(nlse_solver *h, double *U);
 /* enqueue `steps` RK4 steps on the solver's stream (asynchronous) */
 int nlse_step(nlse_solver *h, int steps);
 /* enqueue `steps` steps between two HIP events on the solver's stream,
@@ -305,6 +316,9 @@ void nlse_batch_destroy(nlse_batch *b);
 long long nlse_batch_points(const nlse_batch *b);
 int nlse_batch_set_state(nlse_batch *b, int p, const double *Ur, const double *Ui, const double *V);
 int nlse_batch_get_state(nlse_batch *b, int p, double *Ur, double *Ui);
+/* interleaved complex arrays (see nlse_set_state_z) */
+int nlse_batch_set_state_z(nlse_batch *b, int p, const double *U, const double *V);
+int nlse_batch_get_state_z(nlse_batch *b, int p, double *U);
 int nlse_batch_step(nlse_batch *b, int steps);
 int nlse_batch_step_timed(nlse_batch *b, int steps, double *ms);
 int nlse_batch_sync(nlse_batch *b);

@@ -74,6 +74,18 @@ def lib():
     L.nlse_get_state.argtypes = [C.c_void_p, _D, _D]
     L.nlse_get_state_f.restype = C.c_int
     L.nlse_get_state_f.argtypes = [C.c_void_p, _F, _F]
+    _vp = C.c_void_p
+    L.nlse_set_state_z.restype = C.c_int
+    L.nlse_set_state_z.argtypes = [_vp, _vp, _vp]
+    L.nlse_get_state_z.restype = C.c_int
+    L.nlse_get_state_z.argtypes = [_vp, _vp]
+    L.nlse_batch_set_state_z.restype = C.c_int
+    L.nlse_batch_set_state_z.argtypes = [_vp, C.c_int, _vp, _vp]
+    L.nlse_batch_get_state_z.restype = C.c_int
+    L.nlse_batch_get_state_z.argtypes = [_vp, C.c_int, _vp]
+    L.nlse_take_steps_z.restype = C.c_int
+    L.nlse_take_steps_z.argtypes = ([C.c_int] + [_vp] * 3 + [C.c_double] * 3 + [C.c_int] * 2 + [C.c_double] +
+                                    [C.c_int] * 5)
     L.nlse_step.restype = C.c_int
     L.nlse_step.argtypes = [C.c_void_p, C.c_int]
     L.nlse_step_timed.restype = C.c_int
@@ -201,13 +213,6 @@ def _tail(shape):
     raise ValueError("U must be 1-, 2- or 3-dimensional")
 
 
-def _cplx(re_, im_):
-    out = np.empty(re_.shape, np.complex128)
-    out.real = re_
-    out.imag = im_
-    return out
-
-
 def take_steps(U, V, s, a, h2, BC, chunk_size, k, precision=2, method=1):
     """One chunk through NLSE{1,2,3}D_TAKE_STEPS_HIP[_F].
 
@@ -220,32 +225,16 @@ def take_steps(U, V, s, a, h2, BC, chunk_size, k, precision=2, method=1):
     V = np.asarray(V, dtype=np.float64)
     if V.shape != U.shape:
         raise ValueError(f"V shape {V.shape} differs from U shape {U.shape}")
-    dim = U.ndim
     tail = _tail(U.shape)
-    L = lib()
-    if precision == 2:
-        ur = np.ascontiguousarray(U.real, dtype=np.float64)
-        ui = np.ascontiguousarray(U.imag if np.iscomplexobj(U) else np.zeros(U.shape), dtype=np.float64)
-        v = np.ascontiguousarray(V)
-        outr = np.empty(U.shape)
-        outi = np.empty(U.shape)
-        _check(getattr(L, f"NLSE{dim}D_TAKE_STEPS_HIP")(
-            _p(ur, C.c_double), _p(ui, C.c_double), _p(v, C.c_double), _p(outr, C.c_double),
-            _p(outi, C.c_double), float(s), float(a), float(h2), int(BC), int(chunk_size), float(k),
-            *tail, int(method)))
-        return _cplx(outr, outi)
-    if precision != 1:
+    if precision not in (1, 2):
         raise ValueError("precision must be 1 (single) or 2 (double)")
-    ur = np.ascontiguousarray(U.real, dtype=np.float32)
-    ui = np.ascontiguousarray(U.imag if np.iscomplexobj(U) else np.zeros(U.shape), dtype=np.float32)
-    v = np.ascontiguousarray(V, dtype=np.float32)
-    outr = np.empty(U.shape, np.float32)
-    outi = np.empty(U.shape, np.float32)
-    f32 = lambda x: float(np.float32(x))
-    _check(getattr(L, f"NLSE{dim}D_TAKE_STEPS_HIP_F")(
-        _p(ur, C.c_float), _p(ui, C.c_float), _p(v, C.c_float), _p(outr, C.c_float), _p(outi, C.c_float),
-        f32(s), f32(a), f32(h2), int(BC), int(chunk_size), f32(k), *tail, int(method)))
-    return _cplx(outr.astype(np.float64), outi.astype(np.float64))
+    u = np.ascontiguousarray(U, dtype=np.complex128)
+    v = np.ascontiguousarray(V)
+    out = np.empty(U.shape, np.complex128)
+    _check(lib().nlse_take_steps_z(U.ndim, u.ctypes.data, v.ctypes.data, out.ctypes.data, float(s), float(a),
+                                   float(h2), int(BC), int(chunk_size), float(k), *tail, *(1,) * (3 - len(tail)),
+                                   int(method), int(precision)))
+    return out
 
 
 def _v2(dim):
@@ -347,21 +336,18 @@ class Solver:
         U = np.asarray(U)
         if U.shape != self.shape:
             raise ValueError("shape mismatch")
-        ur = np.ascontiguousarray(U.real, dtype=np.float64)
-        ui = np.ascontiguousarray(U.imag if np.iscomplexobj(U) else np.zeros(U.shape), dtype=np.float64)
-        vp = None
+        u = np.ascontiguousarray(U, dtype=np.complex128)
+        v = None
         if V is not None:
             v = np.ascontiguousarray(V, dtype=np.float64)
             if v.shape != self.shape:
                 raise ValueError("shape mismatch")
-            vp = _p(v, C.c_double)
-        _check(self._lib.nlse_set_state(self._h, _p(ur, C.c_double), _p(ui, C.c_double), vp))
+        _check(self._lib.nlse_set_state_z(self._h, u.ctypes.data, v.ctypes.data if v is not None else None))
 
     def state(self):
-        outr = np.empty(self.shape)
-        outi = np.empty(self.shape)
-        _check(self._lib.nlse_get_state(self._h, _p(outr, C.c_double), _p(outi, C.c_double)))
-        return _cplx(outr, outi)
+        out = np.empty(self.shape, np.complex128)
+        _check(self._lib.nlse_get_state_z(self._h, out.ctypes.data))
+        return out
 
     def step(self, steps):
         _check(self._lib.nlse_step(self._h, int(steps)))
@@ -597,19 +583,14 @@ class Batch:
         U = np.asarray(U)
         if U.shape != self.shapes[p]:
             raise ValueError("shape mismatch")
-        ur = np.ascontiguousarray(U.real, dtype=np.float64)
-        ui = np.ascontiguousarray(U.imag if np.iscomplexobj(U) else np.zeros(U.shape), dtype=np.float64)
-        vp = None
-        if V is not None:
-            v = np.ascontiguousarray(V, dtype=np.float64)
-            vp = _p(v, C.c_double)
-        _check(self._lib.nlse_batch_set_state(self._h, int(p), _p(ur, C.c_double), _p(ui, C.c_double), vp))
+        u = np.ascontiguousarray(U, dtype=np.complex128)
+        v = np.ascontiguousarray(V, dtype=np.float64) if V is not None else None
+        _check(self._lib.nlse_batch_set_state_z(self._h, int(p), u.ctypes.data, v.ctypes.data if v is not None else None))
 
     def state(self, p):
-        outr = np.empty(self.shapes[p])
-        outi = np.empty(self.shapes[p])
-        _check(self._lib.nlse_batch_get_state(self._h, int(p), _p(outr, C.c_double), _p(outi, C.c_double)))
-        return _cplx(outr, outi)
+        out = np.empty(self.shapes[p], np.complex128)
+        _check(self._lib.nlse_batch_get_state_z(self._h, int(p), out.ctypes.data))
+        return out
 
     def step(self, steps):
         _check(self._lib.nlse_batch_step(self._h, int(steps)))

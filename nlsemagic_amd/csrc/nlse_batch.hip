@@ -312,43 +312,37 @@ void nlse_batch_destroy(nlse_batch* b)
 
 long long nlse_batch_points(const nlse_batch* b) { return b ? b->ntot : 0; }
 
+// problem p's state; Y0, ktot and Y1 hold nothing between steps
+static StateRef state_ref(const nlse_batch* b, int p)
+{
+    const long o = b->off[p];
+    const size_t e = b->prec == 2 ? 16 : 8;
+    return StateRef{(char*)b->U + e * o, b->Ulo ? (char*)b->Ulo + e * o : nullptr, (char*)b->V + e / 2 * o, b->prec,
+                    (long)b->N[p] * b->M[p], b->Y0, b->acc, b->Y1, b->stream};
+}
+
 int nlse_batch_set_state(nlse_batch* b, int p, const double* Ur, const double* Ui, const double* V)
 {
     if (!b || !Ur || p < 0 || p >= b->nprob) return fail(NLSE_EINVAL, "bad argument");
-    const long n = (long)b->N[p] * b->M[p], o = b->off[p];
-    if (b->prec == 2) {
-        if (V) HIPCHK(hipMemcpyAsync((double*)b->V + o, V, sizeof(double) * n, hipMemcpyHostToDevice, b->stream));
-        return upload_planes<double>(Ur, Ui, (double2*)b->U + o, (double*)b->Y0, n, b->stream);
-    }
-    std::vector<float> hr(n), hi(n, 0.f), lr(n), li(n, 0.f);
-    split_hilo(Ur, hr.data(), lr.data(), n);
-    if (Ui) split_hilo(Ui, hi.data(), li.data(), n);
-    if (V) {
-        std::vector<float> v(n);
-        for (long q = 0; q < n; ++q) v[q] = (float)V[q];
-        HIPCHK(hipMemcpyAsync((float*)b->V + o, v.data(), sizeof(float) * n, hipMemcpyHostToDevice, b->stream));
-        HIPCHK(hipStreamSynchronize(b->stream));
-    }
-    int rc = upload_planes<float>(hr.data(), hi.data(), (float2*)b->U + o, (float*)b->Y0, n, b->stream);
-    if (rc == NLSE_OK) rc = upload_planes<float>(lr.data(), li.data(), (float2*)b->Ulo + o, (float*)b->Y0, n, b->stream);
-    return rc;
+    return state_put<double>(state_ref(b, p), HostState<double>{nullptr, Ur, Ui, V}, true);
+}
+
+int nlse_batch_set_state_z(nlse_batch* b, int p, const double* U, const double* V)
+{
+    if (!b || !U || p < 0 || p >= b->nprob) return fail(NLSE_EINVAL, "bad argument");
+    return state_put<double>(state_ref(b, p), HostState<double>{U, nullptr, nullptr, V}, true);
 }
 
 int nlse_batch_get_state(nlse_batch* b, int p, double* Ur, double* Ui)
 {
     if (!b || !Ur || !Ui || p < 0 || p >= b->nprob) return fail(NLSE_EINVAL, "bad argument");
-    const long n = (long)b->N[p] * b->M[p], o = b->off[p];
-    if (b->prec == 2) return download_planes<double>((const double2*)b->U + o, Ur, Ui, (double*)b->Y0, n, b->stream);
-    std::vector<float> hr(n), hi(n), lr(n), li(n);
-    int rc = download_planes<float>((const float2*)b->U + o, hr.data(), hi.data(), (float*)b->Y0, n, b->stream);
-    if (rc == NLSE_OK)
-        rc = download_planes<float>((const float2*)b->Ulo + o, lr.data(), li.data(), (float*)b->Y0, n, b->stream);
-    if (rc != NLSE_OK) return rc;
-    for (long q = 0; q < n; ++q) {
-        Ur[q] = (double)hr[q] + (double)lr[q];
-        Ui[q] = (double)hi[q] + (double)li[q];
-    }
-    return NLSE_OK;
+    return state_get<double>(state_ref(b, p), nullptr, Ur, Ui);
+}
+
+int nlse_batch_get_state_z(nlse_batch* b, int p, double* U)
+{
+    if (!b || !U || p < 0 || p >= b->nprob) return fail(NLSE_EINVAL, "bad argument");
+    return state_get<double>(state_ref(b, p), U, nullptr, nullptr);
 }
 
 int nlse_batch_step(nlse_batch* b, int steps)

@@ -239,13 +239,246 @@ int d2h_pageable(void* dst, const void* src, size_t bytes, hipStream_t st)
     return NLSE_OK;
 }
 
-void split_hilo(const double* x, float* hi, float* lo, long n)
+// ---- states between host arrays and the device
+
+namespace {
+
+// Point p of a host state: interleaved values in one or two pieces (points
+// below `cut` at a, the others at b), or planes a and b (b null: zero).
+template <typename S> struct Pieces {
+    S *a, *b;
+    long cut;  // < 0: planes
+};
+
+template <typename S> __device__ __forceinline__ c2<S> piece_get(const Pieces<const S>& s, long p)
 {
-    for (long p = 0; p < n; ++p) {
-        hi[p] = (float)x[p];
-        lo[p] = (float)(x[p] - (double)hi[p]);
+    if (s.cut < 0) return mk<S>(s.a[p], s.b ? s.b[p] : (S)0);
+    return p < s.cut ? ((const c2<S>*)s.a)[p] : ((const c2<S>*)s.b)[p - s.cut];
+}
+template <typename S> __device__ __forceinline__ void piece_put(const Pieces<S>& s, long p, c2<S> v)
+{
+    if (s.cut < 0) {
+        s.a[p] = v.x;
+        s.b[p] = v.y;
+    } else if (p < s.cut) {
+        ((c2<S>*)s.a)[p] = v;
+    } else {
+        ((c2<S>*)s.b)[p - s.cut] = v;
     }
 }
+
+// host values (S) -> a state of T: rounded, or split into hi + lo for a
+// compensated one (hi = float(x), lo = float(x - hi)); V rounded.  src and Vsrc
+// may be pinned host memory.
+template <typename S, typename T>
+__global__ __launch_bounds__(256) void put_state_kernel(Pieces<const S> src, const S* __restrict__ Vsrc,
+                                                        c2<T>* __restrict__ u, c2<T>* __restrict__ lo,
+                                                        T* __restrict__ V, long n)
+{
+    const long p = (long)blockIdx.x * 256 + threadIdx.x;
+    if (p >= n) return;
+    if (src.a) {
+        const c2<S> x = piece_get<S>(src, p);
+        const c2<T> h = mk<T>((T)x.x, (T)x.y);
+        u[p] = h;
+        if (lo) lo[p] = mk<T>((T)(x.x - (S)h.x), (T)(x.y - (S)h.y));
+    }
+    if (Vsrc) V[p] = (T)Vsrc[p];
+}
+
+template <typename S, typename T>
+__global__ __launch_bounds__(256) void get_state_kernel(const c2<T>* __restrict__ u, const c2<T>* __restrict__ lo,
+                                                        Pieces<S> dst, long n)
+{
+    const long p = (long)blockIdx.x * 256 + threadIdx.x;
+    if (p >= n) return;
+    const c2<T> h = u[p];
+    c2<S> x = mk<S>((S)h.x, (S)h.y);
+    if (lo) {
+        const c2<T> l = lo[p];
+        x.x = x.x + (S)l.x;
+        x.y = x.y + (S)l.y;
+    }
+    piece_put<S>(dst, p, x);
+}
+
+template <typename S>
+hipError_t put_kernel(const StateRef& h, Pieces<const S> src, const S* V)
+{
+    const dim3 g((unsigned)((h.n + 255) / 256));
+    if constexpr (std::is_same<S, double>::value) {
+        if (h.prec == 2) {
+            hipLaunchKernelGGL((put_state_kernel<S, double>), g, dim3(256), 0, h.st, src, V, (double2*)h.u,
+                               (double2*)nullptr, (double*)h.V, h.n);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((put_state_kernel<S, float>), g, dim3(256), 0, h.st, src, V, (float2*)h.u, (float2*)h.lo,
+                       (float*)h.V, h.n);
+    return hipGetLastError();
+}
+
+template <typename S> hipError_t get_kernel(const StateRef& h, Pieces<S> dst)
+{
+    const dim3 g((unsigned)((h.n + 255) / 256));
+    if constexpr (std::is_same<S, double>::value) {
+        if (h.prec == 2) {
+            hipLaunchKernelGGL((get_state_kernel<S, double>), g, dim3(256), 0, h.st, (const double2*)h.u,
+                               (const double2*)nullptr, dst, h.n);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((get_state_kernel<S, float>), g, dim3(256), 0, h.st, (const float2*)h.u, (const float2*)h.lo,
+                       dst, h.n);
+    return hipGetLastError();
+}
+
+// States of up to this many bytes of host arrays go through one pinned block
+// that the conversion kernel reads or writes over PCIe: a launch and a host
+// copy in place of two or three DMA copies with their own submissions.  FP64
+// upload of U and V / download: 2048 points 31 / 23 -> 17 / 14 us, 32768
+// points 223 / 81 -> 44 / 35, 131072 points 189 / 127 -> 142 / 138; at 262144
+// points (6 and 4 MB) the pinned chunks and the DMA engine are as fast.
+constexpr size_t DIRECT_MAX = PinnedBlock::SIZE;
+
+std::mutex g_pin_mu;
+std::vector<char*> g_pin_free;
+int g_pin_made = 0;
+constexpr int PIN_BLOCKS = 16;
+
+}  // namespace
+
+PinnedBlock::PinnedBlock() : p_(nullptr)
+{
+    std::lock_guard<std::mutex> lk(g_pin_mu);
+    if (!g_pin_free.empty()) {
+        p_ = g_pin_free.back();
+        g_pin_free.pop_back();
+    } else if (g_pin_made < PIN_BLOCKS) {
+        void* q = nullptr;
+        if (hipHostMalloc(&q, SIZE, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+            ++g_pin_made;
+            p_ = (char*)q;
+        } else {
+            (void)hipGetLastError();
+        }
+    }
+}
+PinnedBlock::~PinnedBlock()
+{
+    if (!p_) return;
+    std::lock_guard<std::mutex> lk(g_pin_mu);
+    g_pin_free.push_back(p_);
+}
+
+template <typename S> int state_put(const StateRef& h, const HostState<S>& src, bool wait)
+{
+    const size_t pb = sizeof(S) * (size_t)h.n;  // bytes of one plane
+    const bool have = src.z || src.r;
+    const size_t total = (have ? 2 * pb : 0) + (src.V ? pb : 0);
+    if (total <= DIRECT_MAX) {
+        PinnedBlock blk;
+        if (char* q = blk.get()) {
+            Pieces<const S> pc{nullptr, nullptr, -1};
+            const S* Vp = nullptr;
+            if (src.z) {
+                std::memcpy(q, src.z, 2 * pb);
+                pc = {(const S*)q, nullptr, h.n};
+            } else if (src.r) {
+                std::memcpy(q, src.r, pb);
+                if (src.i) std::memcpy(q + pb, src.i, pb);
+                pc = {(const S*)q, src.i ? (const S*)(q + pb) : nullptr, -1};
+            }
+            if (src.V) {
+                std::memcpy(q + (have ? 2 * pb : 0), src.V, pb);
+                Vp = (const S*)(q + (have ? 2 * pb : 0));
+            }
+            HIPCHK(put_kernel<S>(h, pc, Vp));
+            HIPCHK(hipStreamSynchronize(h.st));  // the block goes back to the pool
+            return NLSE_OK;
+        }
+    }
+    int rc = NLSE_OK;
+    const bool same = sizeof(S) == 8 && h.prec == 2;  // no conversion
+    if (src.V) {
+        S* const vd = (S*)(same || (sizeof(S) == 4) ? h.V : h.s2);
+        if ((rc = h2d_pageable(vd, src.V, pb, h.st)) != NLSE_OK) return rc;
+        if (vd != h.V) HIPCHK(put_kernel<S>(h, Pieces<const S>{nullptr, nullptr, -1}, vd));
+    }
+    if (src.z && same) {
+        if ((rc = h2d_pageable(h.u, src.z, 2 * pb, h.st)) != NLSE_OK) return rc;
+    } else if (have) {
+        // s1 is a separate buffer only for single-precision states; a double
+        // state's s0 holds both halves
+        S* const a = (S*)h.s0;
+        S* const b = h.prec == 2 ? a + h.n : (S*)h.s1;
+        Pieces<const S> pc{a, b, -1};
+        if (src.z) {
+            const long cut = h.n / 2;
+            if ((rc = h2d_pageable(a, src.z, 2 * sizeof(S) * (size_t)cut, h.st)) != NLSE_OK) return rc;
+            S* const b2 = h.prec == 2 ? a + 2 * cut : b;
+            if ((rc = h2d_pageable(b2, src.z + 2 * cut, 2 * sizeof(S) * (size_t)(h.n - cut), h.st)) != NLSE_OK) return rc;
+            pc = {a, b2, cut};
+        } else {
+            if ((rc = h2d_pageable(a, src.r, pb, h.st)) != NLSE_OK) return rc;
+            if (src.i && (rc = h2d_pageable(b, src.i, pb, h.st)) != NLSE_OK) return rc;
+            if (!src.i) pc.b = nullptr;
+        }
+        HIPCHK(put_kernel<S>(h, pc, (const S*)nullptr));
+    }
+    if (wait) HIPCHK(hipStreamSynchronize(h.st));
+    return NLSE_OK;
+}
+template int state_put<double>(const StateRef&, const HostState<double>&, bool);
+template int state_put<float>(const StateRef&, const HostState<float>&, bool);
+
+template <typename S> int state_get(const StateRef& h, S* z, S* r, S* i)
+{
+    const size_t pb = sizeof(S) * (size_t)h.n;
+    if (2 * pb <= DIRECT_MAX) {
+        PinnedBlock blk;
+        if (char* q = blk.get()) {
+            const Pieces<S> pc = z ? Pieces<S>{(S*)q, nullptr, h.n} : Pieces<S>{(S*)q, (S*)(q + pb), -1};
+            HIPCHK(get_kernel<S>(h, pc));
+            HIPCHK(hipStreamSynchronize(h.st));
+            if (z) {
+                std::memcpy(z, q, 2 * pb);
+            } else {
+                std::memcpy(r, q, pb);
+                std::memcpy(i, q + pb, pb);
+            }
+            return NLSE_OK;
+        }
+    }
+    int rc = NLSE_OK;
+    if (z && sizeof(S) == 8 && h.prec == 2) {
+        rc = d2h_pageable(z, h.u, 2 * pb, h.st);
+    } else {
+        S* const a = (S*)h.s0;
+        const long cut = z ? h.n / 2 : -1;
+        S* const b = h.prec == 2 ? a + (z ? 2 * cut : h.n) : (S*)h.s1;
+        HIPCHK(get_kernel<S>(h, Pieces<S>{a, b, cut}));
+        if (z) {
+            rc = d2h_pageable(z, a, 2 * sizeof(S) * (size_t)cut, h.st);
+            if (rc == NLSE_OK) rc = d2h_pageable(z + 2 * cut, b, 2 * sizeof(S) * (size_t)(h.n - cut), h.st);
+        } else {
+            rc = d2h_pageable(r, a, pb, h.st);
+            if (rc == NLSE_OK) rc = d2h_pageable(i, b, pb, h.st);
+        }
+    }
+    if (rc != NLSE_OK) return rc;
+    HIPCHK(hipStreamSynchronize(h.st));
+    return NLSE_OK;
+}
+template int state_get<double>(const StateRef&, double*, double*, double*);
+template int state_get<float>(const StateRef&, float*, float*, float*);
+
+int upload_planes(const double* Ur, const double* Ui, double2* dst, double* stage, long n, hipStream_t st)
+{
+    const StateRef h{dst, nullptr, nullptr, 2, n, stage, nullptr, nullptr, st};
+    return state_put<double>(h, HostState<double>{nullptr, Ur, Ui, nullptr}, true);
+}
+
 }  // namespace nlse
 
 namespace {
@@ -525,56 +758,24 @@ int step_impl(nlse_solver* h, int steps)
     return enqueue_steps(h, left);
 }
 
-template <typename T>
-int upload(nlse_solver* h, const T* Ur, const T* Ui, const T* V)
+// the staging areas: Y0, ktot and Y1 hold nothing between steps
+StateRef state_ref(const nlse_solver* h)
 {
-    if (V) {
-        const int rc = h2d_pageable(h->V, V, sizeof(T) * (size_t)h->n, h->stream);
-        if (rc != NLSE_OK) return rc;
-    }
-    int rc = upload_planes<T>(Ur, Ui, (c2<T>*)h->U, (T*)h->Y0, h->n, h->stream);
-    if (rc == NLSE_OK && h->Ulo) HIPCHK(hipMemsetAsync(h->Ulo, 0, sizeof(c2<T>) * (size_t)h->n, h->stream));
-    if (rc == NLSE_OK) HIPCHK(hipStreamSynchronize(h->stream));
-    return rc;
+    return StateRef{h->U, h->Ulo, h->V, h->prec, h->n, h->Y0, h->acc, h->Y1, h->stream};
 }
 
-template <typename T>
-int download(nlse_solver* h, T* Ur, T* Ui)
+// values of a reduction that leaves m doubles at its `out`: reduced straight
+// into pinned memory where there is some, else into `dev` and copied
+template <typename F> int fetch(nlse_solver* h, const char* what, int m, double* dev, double* out, F&& launch)
 {
-    return download_planes<T>((const c2<T>*)h->U, Ur, Ui, (T*)h->Y0, h->n, h->stream);
-}
-
-// double planes -> compensated single-precision state (hi, lo)
-int upload_comp(nlse_solver* h, const double* Ur, const double* Ui, const double* V)
-{
-    const long n = h->n;
-    std::vector<float> hr(n), hi(n), lr(n), li(n, 0.f), zero;
-    split_hilo(Ur, hr.data(), lr.data(), n);
-    if (Ui) split_hilo(Ui, hi.data(), li.data(), n);
-    else std::fill(hi.begin(), hi.end(), 0.f);
-    if (V) {
-        std::vector<float> v(n);
-        for (long p = 0; p < n; ++p) v[p] = (float)V[p];
-        const int rv = h2d_pageable(h->V, v.data(), sizeof(float) * (size_t)n, h->stream);
-        if (rv != NLSE_OK) return rv;
-        HIPCHK(hipStreamSynchronize(h->stream));
-    }
-    int rc = upload_planes<float>(hr.data(), hi.data(), (float2*)h->U, (float*)h->Y0, n, h->stream);
-    if (rc == NLSE_OK) rc = upload_planes<float>(lr.data(), li.data(), (float2*)h->Ulo, (float*)h->Y0, n, h->stream);
-    return rc;
-}
-
-int download_comp(nlse_solver* h, double* Ur, double* Ui)
-{
-    const long n = h->n;
-    std::vector<float> hr(n), hi(n), lr(n), li(n);
-    int rc = download_planes<float>((const float2*)h->U, hr.data(), hi.data(), (float*)h->Y0, n, h->stream);
-    if (rc == NLSE_OK) rc = download_planes<float>((const float2*)h->Ulo, lr.data(), li.data(), (float*)h->Y0, n, h->stream);
-    if (rc != NLSE_OK) return rc;
-    for (long p = 0; p < n; ++p) {
-        Ur[p] = (double)hr[p] + (double)lr[p];
-        Ui[p] = (double)hi[p] + (double)li[p];
-    }
+    PinnedBlock blk;
+    double* const d = blk.get() ? (double*)blk.get() : dev;
+    hipError_t e = launch(d);
+    if (e == hipSuccess && d == dev)
+        e = hipMemcpyAsync(out, dev, sizeof(double) * m, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return fail(NLSE_EHIP, std::string(what) + ": " + hipGetErrorString(e));
+    if (d != dev) std::memcpy(out, d, sizeof(double) * m);
     return NLSE_OK;
 }
 
@@ -655,9 +856,10 @@ int take_steps(int dim, const T* Ur, const T* Ui, const T* V, T* Unr, T* Uni, do
     const int prec = sizeof(T) == 8 ? 2 : 1;
     nlse_solver* h = cached_solver(dim, N, M, L, method, prec, BC, s, a, h2, k, &rc);
     if (!h) return rc;
-    if ((rc = upload<T>(h, Ur, Ui, V)) != NLSE_OK) return rc;
+    const StateRef r = state_ref(h);
+    if ((rc = state_put<T>(r, HostState<T>{nullptr, Ur, Ui, V}, false)) != NLSE_OK) return rc;
     if ((rc = step_impl(h, chunk)) != NLSE_OK) return rc;
-    return download<T>(h, Unr, Uni);
+    return state_get<T>(state_ref(h), nullptr, Unr, Uni);
 }
 
 }  // namespace
@@ -704,8 +906,11 @@ int nlse_create(nlse_solver** out, int dim, int N, int M, int L, int method, int
     h->n = (long)N * M * L;
     const size_t eb = elem_bytes(precision) * (size_t)h->n;
     void** bufs[4] = {&h->U, &h->Y0, &h->Y1, &h->acc};
-    for (void** b : bufs)
-        if (dev_malloc(b, eb) != hipSuccess) { nlse_destroy(h); return fail(NLSE_ENOMEM, "hipMalloc failed"); }
+    for (void** b : bufs)  // ktot: one point more, for the second half of a staged state of odd size
+        if (dev_malloc(b, eb + (b == &h->acc ? 16 : 0)) != hipSuccess) {
+            nlse_destroy(h);
+            return fail(NLSE_ENOMEM, "hipMalloc failed");
+        }
     if (dev_malloc(&h->V, eb / 2) != hipSuccess) { nlse_destroy(h); return fail(NLSE_ENOMEM, "hipMalloc failed"); }
     if (dim == 3 && method == 2 && dev_malloc(&h->D, eb) != hipSuccess) {
         nlse_destroy(h);
@@ -767,39 +972,60 @@ void nlse_destroy(nlse_solver* h)
 int nlse_set_state(nlse_solver* h, const double* Ur, const double* Ui, const double* V)
 {
     if (!h || !Ur) return fail(NLSE_EINVAL, "null argument");
-    if (h->prec == 2) return upload<double>(h, Ur, Ui, V);
-    if (h->prec == 3) return upload_comp(h, Ur, Ui, V);
-    std::vector<float> r(h->n), i(h->n, 0.0f), v;
-    for (long p = 0; p < h->n; ++p) r[p] = (float)Ur[p];
-    if (Ui) for (long p = 0; p < h->n; ++p) i[p] = (float)Ui[p];
-    if (V) { v.resize(h->n); for (long p = 0; p < h->n; ++p) v[p] = (float)V[p]; }
-    return upload<float>(h, r.data(), i.data(), V ? v.data() : nullptr);
+    return state_put<double>(state_ref(h), HostState<double>{nullptr, Ur, Ui, V}, true);
+}
+
+int nlse_set_state_z(nlse_solver* h, const double* U, const double* V)
+{
+    if (!h || !U) return fail(NLSE_EINVAL, "null argument");
+    return state_put<double>(state_ref(h), HostState<double>{U, nullptr, nullptr, V}, true);
 }
 
 int nlse_set_state_f(nlse_solver* h, const float* Ur, const float* Ui, const float* V)
 {
     if (!h || !Ur) return fail(NLSE_EINVAL, "null argument");
     if (h->prec != 1) return fail(NLSE_EINVAL, "nlse_set_state_f needs a single-precision (1) solver");
-    return upload<float>(h, Ur, Ui, V);
+    return state_put<float>(state_ref(h), HostState<float>{nullptr, Ur, Ui, V}, true);
 }
 
 int nlse_get_state(nlse_solver* h, double* Ur, double* Ui)
 {
     if (!h || !Ur || !Ui) return fail(NLSE_EINVAL, "null argument");
-    if (h->prec == 2) return download<double>(h, Ur, Ui);
-    if (h->prec == 3) return download_comp(h, Ur, Ui);
-    std::vector<float> r(h->n), i(h->n);
-    int rc = download<float>(h, r.data(), i.data());
-    if (rc != NLSE_OK) return rc;
-    for (long p = 0; p < h->n; ++p) { Ur[p] = r[p]; Ui[p] = i[p]; }
-    return NLSE_OK;
+    return state_get<double>(state_ref(h), nullptr, Ur, Ui);
+}
+
+int nlse_get_state_z(nlse_solver* h, double* U)
+{
+    if (!h || !U) return fail(NLSE_EINVAL, "null argument");
+    return state_get<double>(state_ref(h), U, nullptr, nullptr);
 }
 
 int nlse_get_state_f(nlse_solver* h, float* Ur, float* Ui)
 {
     if (!h || !Ur || !Ui) return fail(NLSE_EINVAL, "null argument");
     if (h->prec != 1) return fail(NLSE_EINVAL, "nlse_get_state_f needs a single-precision (1) solver");
-    return download<float>(h, Ur, Ui);
+    return state_get<float>(state_ref(h), nullptr, Ur, Ui);
+}
+
+int nlse_take_steps_z(int dim, const double* U, const double* V, double* Unew, double s, double a, double h2, int BC,
+                      int chunk_size, double k, int N, int M, int L, int method, int precision)
+{
+    if (!U || !V || !Unew) return fail(NLSE_EINVAL, "null array argument");
+    if (chunk_size < 0) return fail(NLSE_EINVAL, "chunk_size must be >= 0");
+    if (precision != 1 && precision != 2) return fail(NLSE_EINVAL, "precision must be 1 (single) or 2 (double)");
+    if (precision == 1) {  // the single-precision integrators take float scalars
+        s = (float)s;
+        a = (float)a;
+        h2 = (float)h2;
+        k = (float)k;
+    }
+    std::lock_guard<std::mutex> lock(g_cache_mu);
+    int rc = NLSE_OK;
+    nlse_solver* h = cached_solver(dim, N, M, L, method, precision, BC, s, a, h2, k, &rc);
+    if (!h) return rc;
+    if ((rc = state_put<double>(state_ref(h), HostState<double>{U, nullptr, nullptr, V}, false)) != NLSE_OK) return rc;
+    if ((rc = step_impl(h, chunk_size)) != NLSE_OK) return rc;
+    return state_get<double>(state_ref(h), Unew, nullptr, nullptr);
 }
 
 int nlse_step(nlse_solver* h, int steps)
@@ -858,11 +1084,9 @@ int nlse_diagnostics(nlse_solver* h, double* out3)
 {
     if (!h || !out3) return fail(NLSE_EINVAL, "null argument");
     double* d = h->ws;  // result, then 3 * 1024 block partials
-    hipError_t e = launch_diag(h->U, h->Ulo, is_double(h), h->n, d + 3, d, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(out3, d, 3 * sizeof(double), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return fail(NLSE_EHIP, std::string("diagnostics: ") + hipGetErrorString(e));
-    return NLSE_OK;
+    return fetch(h, "diagnostics", 3, d, out3, [&](double* out) {
+        return launch_diag(h->U, h->Ulo, is_double(h), h->n, d + 3, out, h->stream);
+    });
 }
 
 int nlse_energy(nlse_solver* h, double* out4)
@@ -876,11 +1100,11 @@ int nlse_energy(nlse_solver* h, double* out4)
     g.ext[2] = h->M;
     g.s = h->s;
     double* d = h->ws;  // result, then 3 * 1024 block partials
-    hipError_t e = launch_energy(h->U, h->Ulo, h->V, is_double(h), g, d + 3, d, h->stream);
     double r[3];
-    if (e == hipSuccess) e = hipMemcpyAsync(r, d, sizeof(r), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return fail(NLSE_EHIP, std::string("energy: ") + hipGetErrorString(e));
+    const int rc = fetch(h, "energy", 3, d, r, [&](double* out) {
+        return launch_energy(h->U, h->Ulo, h->V, is_double(h), g, d + 3, out, h->stream);
+    });
+    if (rc != NLSE_OK) return rc;
     const double hd = std::pow(h->h2, 0.5 * h->dim);  // the cell volume h^d
     out4[1] = hd * (h->a / h->h2) * r[0];
     out4[2] = hd * r[1];
@@ -937,12 +1161,12 @@ int nlse_kfull(nlse_solver* h, double* out3)
     g.s = h->s;
     g.BC = h->BC;
     double* d = h->ws;  // result, then 6 * 1024 block partials
-    hipError_t e = launch_kfull(h->U, h->Ulo, h->V, h->BC == BC_MSD ? h->acc : nullptr, is_double(h), g, d + 6, d,
-                                h->stream);
     double r[6];
-    if (e == hipSuccess) e = hipMemcpyAsync(r, d, sizeof(r), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return fail(NLSE_EHIP, std::string("kfull: ") + hipGetErrorString(e));
+    const int rc = fetch(h, "kfull", 6, d, r, [&](double* out) {
+        return launch_kfull(h->U, h->Ulo, h->V, h->BC == BC_MSD ? h->acc : nullptr, is_double(h), g, d + 6, out,
+                            h->stream);
+    });
+    if (rc != NLSE_OK) return rc;
     // Lmax = max over G of max over points |x - G|; Bmax by the BC
     double lmax = 0;
     for (int i = 0; i < ng; ++i) {
@@ -1332,7 +1556,7 @@ int NLSE3D_VORTICITY_HIP(const double* Ur, const double* Ui, double lh2, double 
     }
     double2* u = (double2*)buf;
     double* w = buf + 2 * n;
-    int rc = upload_planes<double>(Ur, Ui, u, w, n, st);
+    int rc = upload_planes(Ur, Ui, u, w, n, st);
     hipError_t e = hipSuccess;
     if (rc == NLSE_OK) e = launch_vorticity3d<double>(u, nullptr, L, N, M, lh2, veps, w, w + n, w + 2 * n, w + 3 * n, st);
     double* host[4] = {wx, wy, wz, W};

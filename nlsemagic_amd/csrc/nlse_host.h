@@ -86,62 +86,51 @@ template <typename T> inline void coefs3d(Coefs<T>& c, T s, T a, T h2, T k)
 }
 
 
-// interleave two device planes into a complex array, and back
-template <typename T> __global__ void pack_kernel(const T* __restrict__ r, const T* __restrict__ i, c2<T>* __restrict__ u, long n)
-{
-    const long p = (long)blockIdx.x * 256 + threadIdx.x;
-    if (p < n) u[p] = mk<T>(r[p], i[p]);
-}
+// Where a resident state lives, for moving it to and from host arrays.  The
+// staging areas are device buffers that hold nothing between steps: s0, s1 and
+// s2 of 8 n, 8 n + 16 and 8 n bytes for single-precision states; s0 of 16 n
+// bytes for double ones.
+struct StateRef {
+    void *u, *lo, *V;  // lo: low part of a compensated state, else null
+    int prec;          // 2 double, 1 single, 3 single with a compensated state
+    long n;
+    void *s0, *s1, *s2;
+    hipStream_t st;
+};
 
-template <typename T> __global__ void unpack_kernel(const c2<T>* __restrict__ u, T* __restrict__ r, T* __restrict__ i, long n)
-{
-    const long p = (long)blockIdx.x * 256 + threadIdx.x;
-    if (p < n) {
-        const c2<T> v = u[p];
-        r[p] = v.x;
-        i[p] = v.y;
-    }
-}
+// Host arrays of one state: interleaved complex z, or planes r and i (i may
+// be null for input: zero); V may be null.  S: double or float.
+template <typename S> struct HostState {
+    const S* z;
+    const S *r, *i;
+    const S* V;
+};
 
-// Copies between pageable host memory (the caller's planes) and the device,
-// enqueued on `st`: large ones go through pinned chunks that a pool of host
-// threads fills (or empties) while the DMA engine moves the previous chunk
-// (nlse_capi.hip).  h2d returns once the source has been read (the copy may
-// still be in flight on st); d2h returns once the data is in `dst`.
-int h2d_pageable(void* dst, const void* src, size_t bytes, hipStream_t st);
-int d2h_pageable(void* dst, const void* src, size_t bytes, hipStream_t st);
+// host -> device on h.st.  Returns once the sources have been read; the
+// state may still be in flight on the stream unless `wait`.
+template <typename S> int state_put(const StateRef& h, const HostState<S>& src, bool wait);
+// device -> host (after h.st's earlier work), into z, or into r and i
+template <typename S> int state_get(const StateRef& h, S* z, S* r, S* i);
 
-// host planes -> interleaved device array `dst` of n points, through the
-// device staging area `stage` (>= 2n elements of T); Ui may be null (zero)
-template <typename T>
-int upload_planes(const T* Ur, const T* Ui, c2<T>* dst, T* stage, long n, hipStream_t st)
-{
-    const size_t b = sizeof(T) * (size_t)n;
-    int rc = h2d_pageable(stage, Ur, b, st);
-    if (rc != NLSE_OK) return rc;
-    if (Ui) {
-        rc = h2d_pageable(stage + n, Ui, b, st);
-        if (rc != NLSE_OK) return rc;
-    }
-    else HIPCHK(hipMemsetAsync(stage + n, 0, b, st));
-    hipLaunchKernelGGL((pack_kernel<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, stage, stage + n, dst, n);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(st));
-    return NLSE_OK;
-}
+// A block of pinned host memory that kernels can read and write directly,
+// taken from a bounded pool for the length of one call (null when the pool
+// is exhausted or pinned memory cannot be had: callers then copy)
+class PinnedBlock {
+public:
+    PinnedBlock();
+    ~PinnedBlock();
+    PinnedBlock(const PinnedBlock&) = delete;
+    PinnedBlock& operator=(const PinnedBlock&) = delete;
+    char* get() const { return p_; }
+    static constexpr size_t SIZE = 3u << 20;
 
-template <typename T>
-int download_planes(const c2<T>* src, T* Ur, T* Ui, T* stage, long n, hipStream_t st)
-{
-    const size_t b = sizeof(T) * (size_t)n;
-    hipLaunchKernelGGL((unpack_kernel<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, src, stage, stage + n, n);
-    HIPCHK(hipGetLastError());
-    int rc = d2h_pageable(Ur, stage, b, st);
-    if (rc == NLSE_OK) rc = d2h_pageable(Ui, stage + n, b, st);
-    if (rc != NLSE_OK) return rc;
-    HIPCHK(hipStreamSynchronize(st));
-    return NLSE_OK;
-}
+private:
+    char* p_;
+};
+
+// interleaved planes of n points: host planes -> interleaved device array
+// `dst`, through the device staging area `stage` (>= 2n doubles)
+int upload_planes(const double* Ur, const double* Ui, double2* dst, double* stage, long n, hipStream_t st);
 
 // diagnostics of n points (u, plus ulo for a compensated state) into out[0..2]
 // on the device: sum |U|^2, max Re U, non-finite count; part: 3*1024 doubles
@@ -205,8 +194,5 @@ template <typename T>
 int ic_vortex_ring(c2<T>* u, c2<T>* ulo, const IcGrid& q, int m, double OM, double x0, double y0, double z0,
                    double thetax, double thetay, double thetaz, double vx, double vy, double vz, double phase,
                    double a, double s, double d, int opt_2D, double ea, double eb, hipStream_t st);
-
-// split double planes into the hi + lo single-precision pair of a compensated state
-void split_hilo(const double* x, float* hi, float* lo, long n);
 
 }  // namespace nlse

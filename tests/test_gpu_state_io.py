@@ -1,0 +1,76 @@
+"""States between host arrays and the device: complex arrays and split planes,
+through one pinned block (up to 3 MB of host arrays) and through the staged
+copies above it, for every precision.  Odd counts put an unequal split on the
+two staging areas."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import bits_equal
+
+pytestmark = pytest.mark.gpu
+
+# points whose put (24 B each) or get (16 B) ends below, at and above 3 MB
+SIZES = [3, 401, 131071, 131072, 131073, 196608, 196609, 400001]
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import nlsemagic_amd as nm
+    if nm.device_count() < 1:
+        pytest.fail("no HIP device visible")
+    return nm
+
+
+def _stored(U, prec):
+    """What a state of this precision holds of U, widened to double."""
+    if prec == 2:
+        return U
+    hi = U.astype(np.complex64)
+    lo = (U - hi.astype(np.complex128)).astype(np.complex64)
+    return hi.astype(np.complex128) + (lo.astype(np.complex128) if prec == 3 else 0)
+
+
+@pytest.mark.parametrize("prec", [2, 1, 3])
+@pytest.mark.parametrize("n", SIZES)
+def test_state_round_trip(hip, n, prec):
+    print("CASE", n, prec, flush=True)
+    rng = np.random.default_rng(n + prec)
+    U = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    V = rng.standard_normal(n)
+    exp = _stored(U, prec)
+    sol = hip.Solver((n,), 1, prec, 1, -1.0, 1.0, 0.01, 0.001)
+    sol.set_state(U, V)
+    assert bits_equal(sol.state(), exp)
+    dp = C.POINTER(C.c_double)
+    r, i = np.empty(n), np.empty(n)
+    L = hip.lib()
+    assert L.nlse_get_state(sol._h, r.ctypes.data_as(dp), i.ctypes.data_as(dp)) == 0
+    assert bits_equal(r + 1j * i, exp)
+    sol.set_state(np.zeros(n))
+    r[:], i[:] = U.real, U.imag
+    assert L.nlse_set_state(sol._h, r.ctypes.data_as(dp), i.ctypes.data_as(dp), None) == 0
+    assert bits_equal(sol.state(), exp)
+    assert L.nlse_set_state(sol._h, r.ctypes.data_as(dp), None, None) == 0  # no imaginary part: zero
+    assert bits_equal(sol.state(), _stored(U.real + 0j, prec))
+    # V went with the first upload: the energy of a constant state is its sum
+    sol.fill(1.0)
+    v = V.astype(np.float32).astype(float) if prec != 2 else V
+    assert abs(sol.energy()[2] / 0.1 - (v.sum() + 0.5 * n)) < 1e-9 * n
+    sol.close()
+
+
+@pytest.mark.parametrize("prec", [2, 3])
+def test_batch_state_round_trip(hip, prec):
+    shapes = [(3, 5), (301, 437), (37, 64)]
+    rng = np.random.default_rng(prec)
+    B = hip.Batch(shapes, -1.0, 1.0, 0.01, 0.001, method=1, precision=prec)
+    Us = [rng.standard_normal(s) + 1j * rng.standard_normal(s) for s in shapes]
+    for p, U in enumerate(Us):
+        B.set_state(p, U, np.zeros(U.shape))
+    for p, U in enumerate(Us):
+        assert bits_equal(B.state(p), _stored(U, prec))
+    B.close()
