@@ -325,7 +325,7 @@ int nlse_batch_sync(nlse_batch *b);
 /* per-problem diagnostics, out[3p..3p+2] as for nlse_diagnostics */
 int nlse_batch_diagnostics(nlse_batch *b, double *out);
 /* stage kernel family: 0 LDS tiles (rows 8, 16, 32), 1 row-sweep tiles
- * (rows 8 (default), 12, 16), 2 register strips (3..256-row segments, one
+ * (rows 8, 12, 16; default 16, a whole step per launch), 2 register strips (3..256-row segments, one
  * wave each); see nlse_set_kernel */
 int nlse_batch_set_kernel(nlse_batch *b, int kind, int rows);
 /* stages per launch, kernel kind, rows per tile, persistent grid */

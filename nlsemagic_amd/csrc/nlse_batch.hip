@@ -20,7 +20,11 @@ struct nlse_batch {
     void *U, *Ulo, *Y0, *Y1, *acc, *V;
     void* ubase;     // the allocations U and Y1 started in (they swap after fused steps):
     void* ybase;     // the problem table's buffers 0 and 2
-    double* ws;      // diagnostics: 3 results per problem, then 3 * 1024 block partials
+    // diagnostics: 3 results per problem, then 3 doubles per block partial;
+    // part0 (device): each problem's first partial, maxblocks the most a problem has
+    double* ws;
+    int* part0;
+    int maxblocks;
     void* probs;     // device BatchProb2<T>[nprob]
     int* tile_prob;  // device: problem of each tile
     int ntiles;
@@ -136,8 +140,10 @@ int launch_t(nlse_batch* b, int first, int last, const void* yin, void* out)
     a.first = first;
     a.last = last;
     a.tile = b->tile;
-    a.grid = b->grid;
     a.kernel = b->kern;
+    // no more workgroups than there is work for (strips: one unit per wave)
+    const int need = b->kern == KERNEL_STRIPS ? (b->ntiles + 3) / 4 : b->ntiles;
+    a.grid = std::min(b->grid, 8 * ((need + 7) / 8));
     hipError_t e = launch_batch2d<T>(a, b->stream);
     if (e != hipSuccess) return fail(NLSE_EHIP, std::string("batch launch: ") + hipGetErrorString(e));
     return NLSE_OK;
@@ -249,12 +255,18 @@ int nlse_batch_create(nlse_batch** out, int nprob, const int* N, const int* M, c
         o += (long)N[p] * M[p];
     }
     b->ntot = ntot;
-    b->fuse = 2;
+    // a whole RK4 step per launch on row-sweep tiles of 16 rows, and a grid
+    // of several tiles' worth of workgroups per CU, so that the hardware
+    // evens out the unequal tiles.  Per step, pairs of stages on 8-row tiles
+    // with 4 workgroups per CU -> this: 96 problems of sides 64-512 2SHOC FP64
+    // 268 -> 220 us, FP32c 193 -> 159, CD FP64 203 -> 94, FP32c 138 -> 66; 8
+    // problems 2SHOC FP64 36 -> 32, FP32c 29 -> 25.
+    b->fuse = 4;
     b->kern = KERNEL_ROWS;
-    b->tile = 8;
+    b->tile = 16;
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0);
-    b->grid = 8 * ((cus * 4 + 7) / 8);
+    b->grid = 8 * ((cus * 32 + 7) / 8);
     const size_t eb = (precision == 2 ? 16 : 8) * (size_t)ntot;
     void** bufs[5] = {&b->U, &b->Y0, &b->Y1, &b->acc, &b->V};
     for (int i = 0; i < 5; ++i)
@@ -268,9 +280,20 @@ int nlse_batch_create(nlse_batch** out, int nprob, const int* N, const int* M, c
     }
     b->ubase = b->U;
     b->ybase = b->Y1;
-    if (dev_malloc((void**)&b->ws, sizeof(double) * (3 * 1024 + 3 * (size_t)nprob)) != hipSuccess) {
+    std::vector<int> part0(nprob + 1, 0);
+    for (int p = 0; p < nprob; ++p) {
+        const int nb = diag_blocks((long)N[p] * M[p]);
+        part0[p + 1] = part0[p] + nb;
+        b->maxblocks = std::max(b->maxblocks, nb);
+    }
+    if (dev_malloc((void**)&b->ws, sizeof(double) * 3 * ((size_t)part0[nprob] + nprob)) != hipSuccess ||
+        dev_malloc((void**)&b->part0, sizeof(int) * part0.size()) != hipSuccess) {
         nlse_batch_destroy(b);
         return fail(NLSE_ENOMEM, "hipMalloc failed");
+    }
+    if (hipMemcpy(b->part0, part0.data(), sizeof(int) * part0.size(), hipMemcpyHostToDevice) != hipSuccess) {
+        nlse_batch_destroy(b);
+        return fail(NLSE_EHIP, "copy of the partial table failed");
     }
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess) {
@@ -301,7 +324,7 @@ void nlse_batch_destroy(nlse_batch* b)
     if (!b) return;
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     drop_graphs(b);
-    void* bufs[9] = {b->U, b->Ulo, b->Y0, b->Y1, b->acc, b->V, b->probs, b->tile_prob, b->ws};
+    void* bufs[10] = {b->U, b->Ulo, b->Y0, b->Y1, b->acc, b->V, b->probs, b->tile_prob, b->ws, b->part0};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
@@ -370,14 +393,10 @@ int nlse_batch_diagnostics(nlse_batch* b, double* out)
     if (!b || !out) return fail(NLSE_EINVAL, "null argument");
     double* d = b->ws;
     double* part = d + 3 * (size_t)b->nprob;
-    const size_t eb = b->prec == 2 ? 16 : 8;
-    hipError_t e = hipSuccess;
-    for (int p = 0; p < b->nprob && e == hipSuccess; ++p) {
-        const long n = (long)b->N[p] * b->M[p];
-        const char* u = (const char*)b->U + eb * b->off[p];
-        const char* lo = b->Ulo ? (const char*)b->Ulo + eb * b->off[p] : nullptr;
-        e = launch_diag(u, lo, b->prec == 2, n, part, d + 3 * p, b->stream);
-    }
+    hipError_t e = dbl(b) ? launch_batch_diag<double>((const BatchProb2<double>*)b->probs, b->nprob, role(b, b->U),
+                                                     b->maxblocks, b->part0, part, d, b->stream)
+                          : launch_batch_diag<float>((const BatchProb2<float>*)b->probs, b->nprob, role(b, b->U),
+                                                    b->maxblocks, b->part0, part, d, b->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(out, d, 3 * sizeof(double) * b->nprob, hipMemcpyDeviceToHost, b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);

@@ -1649,7 +1649,7 @@ int group_launch_t(nlse_group* g, int first, int last, int r_yin, int r_out)
     a.first = first;
     a.last = last;
     a.tile = GROUP_ROWS;
-    a.grid = g->grid;
+    a.grid = std::min(g->grid, 8 * ((g->ntiles + 7) / 8));
     a.kernel = KERNEL_ROWS;
     const hipError_t e = launch_batch2d<T>(a, g->stream);
     if (e != hipSuccess) return fail(NLSE_EHIP, std::string("group launch: ") + hipGetErrorString(e));
@@ -1695,7 +1695,7 @@ int nlse_group_create(nlse_group** out, nlse_solver* const* members, int n)
     g->stream = nullptr;
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0);
-    g->grid = 8 * ((cus * 4 + 7) / 8);
+    g->grid = 8 * ((cus * 32 + 7) / 8);  // as a batch's (nlse_batch_create)
     // the members' queued work finishes before the group touches their buffers
     for (nlse_solver* h : g->mem)
         if (hipStreamSynchronize(h->stream) != hipSuccess) {

@@ -22,13 +22,14 @@ constexpr int DIAG_BLOCKS = 1024;
 constexpr int NOALLOC_PARTIALS = 3 * DIAG_BLOCKS;
 static __device__ __align__(256) double scratch[NOALLOC_PARTIALS];
 
+// partial nb of `blocks` blocks over n points
 template <typename T>
-__global__ __launch_bounds__(256) void diag_partial_kernel(const c2<T>* __restrict__ u, const c2<T>* __restrict__ ulo,
-                                                           long n, double* __restrict__ part)
+__device__ __forceinline__ void diag_partial(const c2<T>* __restrict__ u, const c2<T>* __restrict__ ulo, long n,
+                                             int nb, int blocks, double* __restrict__ part)
 {
     __shared__ double s_m[256], s_x[256], s_c[256];
     double m = 0.0, mx = -INFINITY, cnt = 0.0;
-    for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < n; p += (long)gridDim.x * 256) {
+    for (long p = (long)nb * 256 + threadIdx.x; p < n; p += (long)blocks * 256) {
         const c2<T> v = u[p];
         double re = v.x, im = v.y;
         if (ulo) {
@@ -56,13 +57,20 @@ __global__ __launch_bounds__(256) void diag_partial_kernel(const c2<T>* __restri
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        part[3 * blockIdx.x + 0] = s_m[0];
-        part[3 * blockIdx.x + 1] = s_x[0];
-        part[3 * blockIdx.x + 2] = s_c[0];
+        part[3 * nb + 0] = s_m[0];
+        part[3 * nb + 1] = s_x[0];
+        part[3 * nb + 2] = s_c[0];
     }
 }
 
-__global__ __launch_bounds__(256) void diag_fold_kernel(const double* __restrict__ part, int nb, double* __restrict__ out)
+template <typename T>
+__global__ __launch_bounds__(256) void diag_partial_kernel(const c2<T>* __restrict__ u, const c2<T>* __restrict__ ulo,
+                                                           long n, double* __restrict__ part)
+{
+    diag_partial<T>(u, ulo, n, blockIdx.x, gridDim.x, part);
+}
+
+__device__ __forceinline__ void diag_fold(const double* __restrict__ part, int nb, double* __restrict__ out)
 {
     __shared__ double s_m[256], s_x[256], s_c[256];
     double m = 0.0, mx = -INFINITY, cnt = 0.0;
@@ -90,11 +98,55 @@ __global__ __launch_bounds__(256) void diag_fold_kernel(const double* __restrict
     }
 }
 
+__global__ __launch_bounds__(256) void diag_fold_kernel(const double* __restrict__ part, int nb, double* __restrict__ out)
+{
+    diag_fold(part, nb, out);
+}
+
+// the same per problem of a batch, with the blocks each problem has alone:
+// block (x, p) is partial x of problem p, whose partials start at part0[p]
+template <typename T>
+__global__ __launch_bounds__(256) void batch_diag_partial_kernel(const BatchProb2<T>* __restrict__ probs, int r_u,
+                                                                 const int* __restrict__ part0,
+                                                                 double* __restrict__ part)
+{
+    const BatchProb2<T>& P = probs[blockIdx.y];
+    const int b0 = part0[blockIdx.y], nb = part0[blockIdx.y + 1] - b0;
+    if ((int)blockIdx.x >= nb) return;
+    diag_partial<T>(P.buf[r_u], P.ulo, (long)P.N * P.M, blockIdx.x, nb, part + 3 * (long)b0);
+}
+
+__global__ __launch_bounds__(256) void batch_diag_fold_kernel(const double* __restrict__ part,
+                                                              const int* __restrict__ part0, double* __restrict__ out)
+{
+    const int p = blockIdx.x, b0 = part0[p];
+    diag_fold(part + 3 * (long)b0, part0[p + 1] - b0, out + 3 * p);
+}
+
+int diag_blocks(long n) { return (int)std::min<long>(DIAG_BLOCKS, (n + 255) / 256); }
+
+// the diagnostics of every problem of a batch (table `probs`, state in buffer
+// r_u) into out[3p ..]: two launches for all of them instead of two each, with
+// the partials each problem has alone, so the bits are the same; part0: prefix
+// sums of diag_blocks, nprob + 1 values
+template <typename T>
+hipError_t launch_batch_diag(const BatchProb2<T>* probs, int nprob, int r_u, int maxblocks, const int* part0,
+                             double* part, double* out, hipStream_t st)
+{
+    hipLaunchKernelGGL((batch_diag_partial_kernel<T>), dim3(maxblocks, nprob), dim3(256), 0, st, probs, r_u, part0, part);
+    hipLaunchKernelGGL(batch_diag_fold_kernel, dim3(nprob), dim3(256), 0, st, part, part0, out);
+    return hipGetLastError();
+}
+template hipError_t launch_batch_diag<double>(const BatchProb2<double>*, int, int, int, const int*, double*, double*,
+                                              hipStream_t);
+template hipError_t launch_batch_diag<float>(const BatchProb2<float>*, int, int, int, const int*, double*, double*,
+                                             hipStream_t);
+
 // enqueue the reduction of n points at u (+ ulo) into out[0..2] (device);
 // `part` holds 3 * DIAG_BLOCKS doubles
 hipError_t launch_diag(const void* u, const void* ulo, bool dbl, long n, double* part, double* out, hipStream_t st)
 {
-    const int nb = (int)std::min<long>(DIAG_BLOCKS, (n + 255) / 256);
+    const int nb = diag_blocks(n);
     if (dbl)
         hipLaunchKernelGGL((diag_partial_kernel<double>), dim3(nb), dim3(256), 0, st, (const double2*)u,
                            (const double2*)nullptr, n, part);

@@ -136,6 +136,13 @@ int upload_planes(const double* Ur, const double* Ui, double2* dst, double* stag
 // on the device: sum |U|^2, max Re U, non-finite count; part: 3*1024 doubles
 hipError_t launch_diag(const void* u, const void* ulo, bool dbl, long n, double* part, double* out, hipStream_t st);
 
+// the same for every problem of a batch in two launches: part0 (device) holds
+// the prefix sums of diag_blocks(points) of its problems (nprob + 1 values)
+int diag_blocks(long n);
+template <typename T>
+hipError_t launch_batch_diag(const BatchProb2<T>* probs, int nprob, int r_u, int maxblocks, const int* part0,
+                             double* part, double* out, hipStream_t st);
+
 // The kfull reduction (nlse_diag.hip): grid of `dim` axes of extents ext[]
 // (slowest first, n points), c = h^2/a, the nonlinearity s and the BC.
 struct KfGrid {
