@@ -272,14 +272,23 @@ constexpr int BLK_SEG = 256;  // the largest segment: owned points per workgroup
 // One wave per 64 consecutive points: a core of CW = 64 - 2 HW points and a
 // halo of HW = 4 R points (one RK4 step's reach) each side, copies of the
 // neighbouring waves' core points.  A wave runs the four stages of a step on
-// its own: the stage input (and D) of its 64 points goes to a wave-private
-// LDS slice and the stencils (with the reference's boundary rules) read it
-// there, so no workgroup barrier is needed within a step (neighbours by DPP
-// instead ran 6 % slower: the lane shifts of FP64 values cost more than the
-// LDS round trip).  The halo lanes go stale by R points per stage and
-// are refreshed from the neighbours' cores (U and U_lo through LDS, one
-// workgroup barrier) at the end of every step.  The window's outer halo of
+// its own in registers: the neighbours i +- 1 of the stage input (and of D)
+// come from the adjacent lanes (DPP).  The halo lanes go stale by R points per
+// stage and are refreshed from the neighbours' cores (U and U_lo through LDS,
+// one workgroup barrier) at the end of every step.  The window's outer halo of
 // 4 R S points covers the S steps of the launch as in the resident kernel.
+//
+// Only waves that hold point 0 or N-1 run the boundary rules (uniform branch),
+// in the boundary point's lane from values its own wave already has: MSD's
+// partner is the adjacent lane (one division per rule), the one-sided formula
+// reaches three lanes.  The cores are laid out so that the last one holds at
+// least four points of the grid, which keeps that reach inside lanes that are
+// exact through all four stages.
+// Bound: the dependent chain of a stage.  Per RK4 step with 32 (CD) or 16
+// (2SHOC) steps per launch, stencils and boundary rules read from LDS in every
+// wave -> this: N = 2048 MSD CD FP64 1.38 -> 0.90 us, 2SHOC FP64 2.53 -> 1.61
+// us; N = 50021 2SHOC FP32c 2.43 -> 1.49 us.  A wave without an end takes
+// 0.59 (CD FP64) and 0.87 us (2SHOC FP64): the rest is the ends' divisions.
 template <typename T, int METHOD, bool COMP>
 __global__ __launch_bounds__(1024) void block1d_kernel(const c2<T>* __restrict__ uin, c2<T>* __restrict__ uout,
                                                        const c2<T>* __restrict__ loin, c2<T>* __restrict__ loout,
@@ -288,15 +297,16 @@ __global__ __launch_bounds__(1024) void block1d_kernel(const c2<T>* __restrict__
 {
     constexpr int R = (METHOD == 2) ? 2 : 1;
     constexpr int HW = 4 * R, CW = 64 - 2 * HW;
-    constexpr int PAD = 4;  // the boundary formulas reach three points inward
-    // wave-private stage input and D (padding lanes hold values no core
-    // point depends on); window-indexed U and U_lo of the cores, by step parity
-    __shared__ c2<T> sW[16][64 + 2 * PAD];
-    __shared__ c2<T> sWD[(METHOD == 2) ? 16 : 1][(METHOD == 2) ? 64 + 2 * PAD : 1];
+    // window-indexed U and U_lo of the cores, by step parity
     __shared__ c2<T> sX[2][16 * CW];
     __shared__ c2<T> sXL[COMP ? 2 : 1][COMP ? 16 * CW : 1];
     const int o0 = max((int)blockIdx.x * seg - soff, 0), o1 = min((int)(blockIdx.x + 1) * seg - soff, N);
-    const int w0 = max(o0 - halo, 0), w1 = min(o1 + halo, N);
+    const int w1 = min(o1 + halo, N);
+    int w0 = max(o0 - halo, 0);
+    // a window that ends at the grid: its last core holds at least four points
+    // (the first then starts up to three points earlier)
+    const int tail = (w1 - w0) % CW;
+    if (w1 == N && tail > 0 && tail < 4) w0 -= 4 - tail;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nw = (w1 - w0 + CW - 1) / CW;  // waves with a core in the window
@@ -306,11 +316,18 @@ __global__ __launch_bounds__(1024) void block1d_kernel(const c2<T>* __restrict__
     const int ic = i < 0 ? 0 : (i >= N ? N - 1 : i);
     c2<T> U = uin[ic], Lo = COMP ? loin[ic] : mk<T>(0, 0), A = mk<T>(0, 0), Y = U;
     const T Vr = Vg[ic];
-    auto Vl = [&](int gi) { return gi == i ? Vr : Vg[gi]; };
-    auto Yl = [&](int gi) { return sW[w][gi - ib + PAD]; };
-    auto Dl = [&](int gi) { return sWD[METHOD == 2 ? w : 0][gi - ib + PAD]; };
-    auto rhs = make_rhs1d<T, METHOD>(Yl, Vl, Dl, c, N, BC);
-    const bool ingrid = i >= 0 && i < N;
+    const bool edge = ib <= 0 || ib + 63 >= N - 1;  // this wave holds an end of the grid (uniform)
+    const bool bnd = i == 0 || i == N - 1;
+    auto nx = [](c2<T> v) { return lane_shift2<DPP_NEXT, T>(v); };
+    auto pv = [](c2<T> v) { return lane_shift2<DPP_PREV, T>(v); };
+    // one-sided second difference at an end, inward (NLSEmagic1D_CPU.c:60-68);
+    // yn, yp: the stage input at i+1, i-1
+    auto onesided = [&](c2<T> yn, c2<T> yp) {
+        const c2<T> n2 = nx(yn), p2 = pv(yp), n3 = nx(n2), p3 = pv(p2);
+        const bool left = i == 0;
+        const c2<T> q1 = left ? yn : yp, q2 = left ? n2 : p2, q3 = left ? n3 : p3;
+        return mk<T>(-q3.x + 4 * q2.x - 5 * q1.x + 2 * Y.x, -q3.y + 4 * q2.y - 5 * q1.y + 2 * Y.y);
+    };
     // distance of this wave's nearest point from the segment (uniform)
     const int whi = ib + 63;
     const int wdist = whi < o0 ? o0 - whi : (ib > o1 - 1 ? ib - (o1 - 1) : 0);
@@ -323,14 +340,47 @@ __global__ __launch_bounds__(1024) void block1d_kernel(const c2<T>* __restrict__
             // waves with no core in the window, skip the stage
             const bool live = w < nw && wdist <= R * (G - (4 * step + stage - 1));
             if (!live) return;
-            sW[w][PAD + lane] = Y;
-            __builtin_amdgcn_wave_barrier();
-            if constexpr (METHOD == 2) {
-                const c2<T> d = ingrid ? rhs.d_at(i) : mk<T>(0, 0);
-                sWD[w][PAD + lane] = d;
-                __builtin_amdgcn_wave_barrier();
+            const c2<T> yn = nx(Y), yp = pv(Y);
+            const T n = nlin<T>(c.s, Y, Vr);
+            c2<T> f;
+            if constexpr (METHOD == 1) {
+                // NLSEmagic1D_CPU.c:27-30
+                f = mk<T>(-c.ah2 * (yn.y - 2 * Y.y + yp.y) - n * Y.y, c.ah2 * (yn.x - 2 * Y.x + yp.x) + n * Y.x);
+            } else {
+                // D (NLSEmagic1D_CPU.c:150-198), then F (:204-207)
+                c2<T> d = mk<T>((yn.x - 2 * Y.x + yp.x) * c.lh2, (yn.y - 2 * Y.y + yp.y) * c.lh2);
+                if (edge) {
+                    c2<T> db = mk<T>(0, 0);
+                    if (BC == BC_DIRICHLET) {
+                        db = dir_d<T>(Y, Vr, c);
+                    } else if (BC == BC_MSD) {
+                        const T a = msd_col<T>((d.x * Y.x + d.y * Y.y) / (Y.x * Y.x + Y.y * Y.y), i, N);
+                        const T n1 = msd_col<T>(n, i, N);
+                        db = mk<T>((a + c.l_a * (n1 - n)) * Y.x, (a + c.l_a * (n1 - n)) * Y.y);
+                    } else if (BC == BC_ONESIDED) {
+                        const c2<T> o = onesided(yn, yp);
+                        db = mk<T>(o.x * c.lh2, o.y * c.lh2);
+                    }
+                    if (bnd) d = db;
+                }
+                const c2<T> da = nx(d), db = pv(d);
+                f = mk<T>(c.a112 * (da.y + db.y) - c.a76 * d.y - n * Y.y, c.a76 * d.x - c.a112 * (da.x + db.x) + n * Y.x);
             }
-            const c2<T> f = ingrid ? rhs.f_at(i) : mk<T>(0, 0);
+            if (edge) {  // F at the ends (NLSEmagic1D_CPU.c:33-76, 210-253)
+                c2<T> fb = mk<T>(0, 0);
+                if (BC == BC_MSD) {
+                    fb = msd_om<T>(msd_col<T>(msd_rate<T>(f, Y), i, N), Y);
+                } else if (BC == BC_LAP0) {
+                    fb = mk<T>(-n * Y.y, n * Y.x);
+                } else if (BC == BC_ONESIDED) {
+                    const c2<T> o = onesided(yn, yp);
+                    if constexpr (METHOD == 1)
+                        fb = mk<T>(-c.ah2 * o.y - n * Y.y, c.ah2 * o.x + n * Y.x);
+                    else
+                        fb = mk<T>(-c.a * o.y * c.lh2 - n * Y.y, c.a * o.x * c.lh2 + n * Y.x);
+                }
+                if (bnd) f = fb;
+            }
             if constexpr (stage == 1) {
                 A = f;
                 Y = mk<T>(U.x + c.k2 * f.x, U.y + c.k2 * f.y);
@@ -349,16 +399,15 @@ __global__ __launch_bounds__(1024) void block1d_kernel(const c2<T>* __restrict__
                 const T kk = (stage == 2) ? c.k2 : c.k;
                 Y = mk<T>(U.x + kk * f.x, U.y + kk * f.y);
             }
-            __builtin_amdgcn_wave_barrier();  // the slices are read before the next stage rewrites them
         });
         // refresh the halo lanes from the neighbouring waves' cores
         const int par = step & 1;
+        const int x = i - w0;
         if (core && w < nw) {
-            sX[par][i - w0] = U;
-            if constexpr (COMP) sXL[par][i - w0] = Lo;
+            sX[par][x] = U;
+            if constexpr (COMP) sXL[par][x] = Lo;
         }
         __syncthreads();
-        const int x = i - w0;
         if (!core && w < nw && x >= 0 && x < nw * CW && i < w1) {
             U = sX[par][x];
             if constexpr (COMP) Lo = sXL[par][x];
