@@ -11,11 +11,13 @@
 //     all at once at the start, stage input first (every load in flight
 //     together; rows outside the grid load a clamped copy, so every wave
 //     issues the same loads);
-//   - the rows i +- 1, the diagonal corners of the 2SHOC stencil and a row's
-//     own j +- 1 neighbours come from the LDS copy of the stage input (lane
-//     +- 1 of a row's copy costs no VALU moves, unlike DPP shifts of FP64
-//     values), and for 2SHOC D = Lap_CD(Y)/h^2 of rows i +- 1 and columns
-//     j +- 1 from an LDS copy of D;
+//   - the rows i +- 1 and the diagonal corners of the 2SHOC stencil come from
+//     the LDS copy of the stage input, and for 2SHOC D = Lap_CD(Y)/h^2 of rows
+//     i +- 1 from an LDS copy of D.  A row's own j +- 1 neighbours: 2SHOC shifts
+//     lanes (DPP), which takes 4 of its 15 LDS accesses per row and stage away
+//     (1024^2 per step: FP32 19.2 -> 18.1 us, FP32c 20.8 -> 20.0, FP64 30.3 ->
+//     30.0, which then needs no spill); CD reads lane +- 1 of the LDS copy (with
+//     lane shifts FP64 15.8 -> 16.3 us, FP32 equal);
 //   - per stage: D phase, barrier, F phase (each row's F and RK4 update at
 //     once, the new Y in the row's registers), barrier, new Y rows written
 //     to LDS, barrier; the last stage writes its rows to HBM.
@@ -207,7 +209,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 c2<T> dd = z;
                 if (interior(g)) {
                     const c2<T> a = sy(e + 1, 0), b = sy(e - 1, 0);
-                    const c2<T> yp = sy(e, 1), ym = sy(e, -1);  // the row's k +- 1 neighbours from its LDS copy
+                    const c2<T> yp = lane_shift2<DPP_NEXT, T>(yx), ym = lane_shift2<DPP_PREV, T>(yx);
                     dd = mk<T>((a.x + b.x - 4 * yx.x + yp.x + ym.x) * c.lh2, (a.y + b.y - 4 * yx.y + yp.y + ym.y) * c.lh2);
                     if (colbc && !msd) {  // MSD columns: the column pass below
                         c2<T> db = z;
@@ -306,7 +308,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 const T n = nlin<T>(c.s, yx, vx);
                 if constexpr (METHOD == 2) {
                     const c2<T> dc = sd(e, 0), da = sd(e + 1, 0), db = sd(e - 1, 0);
-                    const c2<T> dl = sd(e, 1), dr = sd(e, -1);
+                    const c2<T> dl = lane_shift2<DPP_NEXT, T>(dc), dr = lane_shift2<DPP_PREV, T>(dc);
                     const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
                     ff = mk<T>(-c.a * dc.y + c.a1_12 * (da.y + db.y + dl.y + dr.y)
                                    - c.a1_6h2 * (aa.y + ab.y - 4 * yx.y + ba.y + bb.y) - n * yx.y,
