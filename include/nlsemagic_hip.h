@@ -269,7 +269,7 @@ int nlse_set_fusion(nlse_solver *h, int stages_per_launch);
  * every choice):
  *   kind 0  LDS tiles of 64 columns x 8, 16 or 32 rows
  *   kind 1  row-sweep LDS tiles (one lane per column, DPP neighbours),
- *           8, 12 or 16 (default) rows
+ *           8, 12 or 16 rows (default by grid size: 16 from about 700^2 on)
  *   kind 2  register-marching strips (one wave per strip, no LDS), segments
  *           of 3..256 rows, for 1, 2 or 4 stages per launch
  * 3D 2SHOC, one stage per launch: kind 1 (default) marches planes with D

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
                                                                  ulo);
 }
 
-template <typename T, int METHOD, int FIRST, int LAST, int TI>
+template <typename T, int METHOD, int FIRST, int LAST, int TI, int NW = rows_waves<METHOD, FIRST, LAST, TI>()>
 static hipError_t launch_rows_ti(const StageArgs<T>& a, hipStream_t st)
 {
     constexpr int W = RowsCfg<METHOD, FIRST, LAST, TI>::W;
@@ -128,7 +128,6 @@ static hipError_t launch_rows_ti(const StageArgs<T>& a, hipStream_t st)
     g.map.ntiles = g.tiles_i * g.tiles_j;
     g.map.per_xcd = (g.map.ntiles + 7) / 8;
     const int nwg = g.edge_first_setup();
-    constexpr int NW = rows_waves<METHOD, FIRST, LAST, TI>();
     if constexpr (std::is_same<T, float>::value && LAST == 4) {
         if (a.ulo) {
             hipLaunchKernelGGL((rows2d_kernel<T, METHOD, FIRST, LAST, TI, true, NW>), dim3(nwg), dim3(NW * 64), 0,
@@ -141,9 +140,66 @@ static hipError_t launch_rows_ti(const StageArgs<T>& a, hipStream_t st)
     return hipGetLastError();
 }
 
+// Whole-step tiles by grid size.  A launch with few tiles takes one tile's
+// time, which shorter tiles and more waves cut; once the tiles come in several
+// rounds the work of their halo rows counts instead.  The lines, in tiles per
+// CU of 8, 12 and 16 rows, from a sweep of 12 grids (100^2 to 1024^2, both
+// methods, all precisions, Dirichlet and MSD; per step, 16 rows on 8 waves ->
+// the choice):
+//   8 rows on 16 waves   100^2 CD FP64 6.7 -> 4.7 us, 2SHOC FP64 11.3 -> 8.0
+//                        (MSD 14.4 -> 10.3), 448^2 CD FP32 MSD 7.7 -> 5.2
+//   8 rows on 8 waves    384^2 2SHOC FP64 11.7 -> 9.9, 512^2 2SHOC FP32 10.0 ->
+//                        8.4, 600^2 CD FP32c MSD 8.2 -> 6.6
+//   12 rows on 8 waves   512^2 2SHOC FP64 12.2 -> 10.8
+//   16 rows on 16 waves  600^2 2SHOC FP32 10.2 -> 8.6; 1000 x 100 2SHOC FP64
+//                        10.2 (two of three tiles hold a boundary: 8 rows 12.6)
+//   16 rows on 8 waves   from 700^2 on (8 rows there: 2SHOC FP64 18.0 -> 21.4)
+struct RowsChoice {
+    int rows, waves;
+};
+static RowsChoice rows_choice(int method, bool dbl, int N, int M)
+{
+    const int W = method == 2 ? 48 : 56;
+    const long cols = (M + (M % W == 1) + W - 1) / W;
+    auto tiles = [&](int TI) { return cols * ((N + (N % TI == 1) + TI - 1) / TI); };
+    const long cus = device_cus();
+    if (method == 1) {
+        if (tiles(8) <= 2 * cus) return {8, 16};
+        if (tiles(8) <= 4 * cus) return {8, 8};
+        return {16, 8};
+    }
+    if (tiles(8) <= cus) return {8, 16};
+    if (cols <= 3 && tiles(16) <= cus) return {16, 16};
+    if (4 * tiles(8) <= (dbl ? 9 : 12) * cus) return {8, 8};
+    if (dbl && tiles(12) <= 2 * cus) return {12, 8};
+    if (!dbl && tiles(16) <= 2 * cus) return {16, 16};
+    return {16, 8};
+}
+
+int default_rows2d(int method, bool dbl, int N, int M) { return rows_choice(method, dbl, N, M).rows; }
+
+// a whole step on tiles of a.tile rows: the waves of the choice where it has
+// these rows, else 16 waves while there is at most one tile per CU
+template <typename T, int METHOD>
+static hipError_t launch_rows_step(const StageArgs<T>& a, hipStream_t st)
+{
+    const RowsChoice c = rows_choice(METHOD, std::is_same<T, double>::value, a.N, a.M);
+    const int W = METHOD == 2 ? 48 : 56;
+    const int NW = c.rows == a.tile ? c.waves
+                                    : ((long)((a.N + a.tile - 1) / a.tile) * ((a.M + W - 1) / W) <= device_cus() ? 16 : 8);
+    switch (a.tile) {
+    case 12: return launch_rows_ti<T, METHOD, 1, 4, 12, 8>(a, st);
+    case 16:
+        return NW == 16 ? launch_rows_ti<T, METHOD, 1, 4, 16, 16>(a, st) : launch_rows_ti<T, METHOD, 1, 4, 16, 8>(a, st);
+    default:
+        return NW == 16 ? launch_rows_ti<T, METHOD, 1, 4, 8, 16>(a, st) : launch_rows_ti<T, METHOD, 1, 4, 8, 8>(a, st);
+    }
+}
+
 template <typename T, int METHOD, int FIRST, int LAST>
 static hipError_t launch_rows(const StageArgs<T>& a, hipStream_t st)
 {
+    if constexpr (FIRST == 1 && LAST == 4) return launch_rows_step<T, METHOD>(a, st);
     switch (a.tile) {
     case 12: return launch_rows_ti<T, METHOD, FIRST, LAST, 12>(a, st);
     case 16: return launch_rows_ti<T, METHOD, FIRST, LAST, 16>(a, st);

@@ -17,8 +17,6 @@
 // Neighbour reads of the per-point kernels go through the L1/L2 caches: a
 // wavefront covers 64 consecutive k, so every plane and row neighbour is a
 // coalesced line read.
-#include <atomic>
-
 #include "nlse3d_cdpair.h"
 #include "nlse3d_march.h"
 #include "nlse3d_shocpair.h"
@@ -215,21 +213,6 @@ __global__ __launch_bounds__((TJ + 4) * 64) void shocpair3d_kernel(const c2<T>* 
         ShocPair<T, FIRST, TJ, MSD, Lds>(sm, i0, j0, k0, g, yin, u, acc, yout, V, c, BC, ulo).run();
     else
         ShocPair<T, FIRST, TJ, false, Lds>(sm, i0, j0, k0, g, yin, u, acc, yout, V, c, BC, ulo).run();
-}
-
-// compute units of the current device
-static int device_cus()
-{
-    static std::atomic<int> cus{0};
-    int n = cus.load(std::memory_order_relaxed);
-    if (n == 0) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        cus.store(n, std::memory_order_relaxed);
-    }
-    return n;
 }
 
 // Planes per chunk of a pair launch with `cols` tiles per plane, H halo planes

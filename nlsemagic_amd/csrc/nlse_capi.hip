@@ -31,6 +31,21 @@ int set_error(int code, const std::string& msg)
 
 std::atomic<long long> g_allocs{0};
 
+// compute units of the current device
+int device_cus()
+{
+    static std::atomic<int> cus{0};
+    int n = cus.load(std::memory_order_relaxed);
+    if (n == 0) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        cus.store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
 hipError_t dev_malloc_raw(void** p, size_t bytes)
 {
     ++g_allocs;
@@ -938,7 +953,7 @@ int nlse_create(nlse_solver** out, int dim, int N, int M, int L, int method, int
     h->fuse = (dim == 1) ? 1 : (dim == 2 ? 4 : 2);
     h->kern = KERNEL_ROWS;         // the fastest family on a 1024^2 grid and for 3D 2SHOC
     // 3D: plane-march rows; 1D: steps per launch (the fastest on N = 2048)
-    h->tile = (dim == 3) ? 4 : (dim == 1 ? (method == 2 ? 16 : 32) : 16);
+    h->tile = (dim == 3) ? 4 : (dim == 1 ? (method == 2 ? 16 : 32) : default_rows2d(method, precision == 2, N, M));
     set_params(h, BC, s, a, h2, k);
     // a defined initial state: zero field and potential, cleared on the
     // solver's own stream (a null-stream memset is not ordered with it and

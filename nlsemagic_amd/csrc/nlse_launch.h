@@ -31,6 +31,11 @@ template <typename T> struct StageArgs {
 //                  1, 2 or 4 stages per launch (nlse2d_strip.h)
 enum { KERNEL_TILES = 0, KERNEL_ROWS = 1, KERNEL_STRIPS = 2 };
 
+// compute units of the current device (256 where it cannot be asked)
+int device_cus();
+// rows per row-sweep tile a 2D solver of this shape starts with (8, 12 or 16)
+int default_rows2d(int method, bool dbl, int N, int M);
+
 template <typename T> hipError_t launch_stage1d(const StageArgs<T>& a, hipStream_t st);
 template <typename T> hipError_t launch_stage2d(const StageArgs<T>& a, hipStream_t st);
 template <typename T> hipError_t launch_stage3d(const StageArgs<T>& a, hipStream_t st);
