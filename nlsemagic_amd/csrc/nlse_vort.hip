@@ -16,7 +16,7 @@
 // is 0 as in the reference's zero-initialised outputs.  Single-precision
 // states are widened (hi + lo) to double first.
 //
-// One kernel, no scratch: a workgroup owns TJ rows (j) x 60 columns (k) and
+// One kernel, no scratch: a workgroup owns TJ rows (j) x 56 or 60 columns (k) and
 // marches along i over a chunk of planes.  Lane l is column k0 - 2 + l;
 // extended row e is row j0 - 2 + e.  At step p a row takes U of plane p
 // (loaded two steps ahead), the rows next to the owned ones and the owned ones
@@ -31,10 +31,10 @@
 //
 // Rows and planes inside the grid, in tiles without column 0 or M-1, run
 // central differences only (uniform branch); the others select operands per
-// lane, without branches.  Bound: HBM at 256^3 (4.8 TB/s on the 48 B a point
-// needs; a large copy reaches 5.06).  Per call, 16 rows on 16 waves with a
+// lane, without branches.  Bound: HBM at 256^3 (the 48 B a point needs take
+// 159 us at the rate of a large copy).  Per call, 16 rows on 16 waves with a
 // branch per difference and loads widened at once -> this: 256^3 FP64 244 ->
-// 168 us, FP32 275 -> 169, FP32c 333 -> 167; 201 x 180 x 190 FP64 150 -> 99;
+// 151 us, FP32 275 -> 149, FP32c 333 -> 158; 201 x 180 x 190 FP64 150 -> 99;
 // 64^3 FP64 68 -> 14.
 #include "nlse2d_strip.h"
 #include "nlse_host.h"
@@ -65,6 +65,7 @@ template <typename T, bool COMP> struct Raw {
 
 struct VortMarch {
     int IC;                 // planes per chunk
+    int kw;                 // owned columns, at most 60
     int tj, tk, ti;         // tiles along j, k and chunks along i
     int per_xcd;            // workgroups per XCD
 };
@@ -96,7 +97,7 @@ struct VortTile {
     const Dims3& g;
     double *wx, *wy, *wz, *W;
     const int i0, iend, j0, k, lane;
-    const bool kin, kb, ktile;  // column in the grid, on its boundary; the tile holds a boundary column (uniform)
+    const bool kout, kb, ktile;  // an owned column in the grid, a column on its boundary; the tile holds a boundary column (uniform)
 
     template <int LV> __device__ __forceinline__ void init(Row<LV>& R, int e) const
     {
@@ -212,7 +213,7 @@ struct VortTile {
                     double ox = vzy - vyz, oy = vxz - vzx, oz = vyx - vxy;
                     double on = sqrt(ox * ox + oy * oy + oz * oz);
                     if (!ok) ox = oy = oz = on = 0;
-                    if (lane >= 2 && lane <= 61 && kin) {
+                    if (kout) {
                         const long pp = (long)cp * g.si + R.ro;
                         // streaming stores: the four outputs are not read
                         // again by this launch (3.8 % faster per call at 256^3)
@@ -255,12 +256,12 @@ __global__ __launch_bounds__((TJ + 1) * 64) void vort_march_kernel(const c2<T>* 
     if (t >= vm.tj * vm.tk * vm.ti) return;
     const int kt = t % vm.tk, rest = t / vm.tk;
     const int jt = rest % vm.tj, ci = rest / vm.tj;
-    const int i0 = ci * vm.IC, k0 = kt * 60, lane = threadIdx.x & 63;
+    const int i0 = ci * vm.IC, k0 = kt * vm.kw, lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int k = k0 - 2 + lane;
     using Tile = VortTile<T, COMP, TJ>;
     const Tile tile{sm, u, ulo, lh2, veps, g, wx, wy, wz, W, i0, min(i0 + vm.IC, g.L), jt * TJ, k, lane,
-                    k >= 0 && k < g.M, k == 0 || k == g.M - 1, k0 - 2 <= 0 || k0 - 2 + 63 >= g.M - 1};
+                    k >= 0 && k < g.M && lane >= 2 && lane < 2 + vm.kw, k == 0 || k == g.M - 1, k0 - 2 <= 0 || k0 - 2 + 63 >= g.M - 1};
     if (w < TJ) {
         typename Tile::template Row<2> r;
         tile.init(r, 2 + w);
@@ -285,7 +286,7 @@ hipError_t launch_vorticity3d(const c2<T>* u, const c2<T>* ulo, int L, int N, in
                               double* wx, double* wy, double* wz, double* W, hipStream_t st)
 {
     // 7 owned rows on 8 waves, two workgroups per CU (15 rows: 256^3
-    // FP64 179 us, against 168)
+    // FP64 179 us, against 168, both with 60 columns)
     constexpr int TJ = 7;
     Dims3 g;
     g.L = L;
@@ -295,8 +296,12 @@ hipError_t launch_vorticity3d(const c2<T>* u, const c2<T>* ulo, int L, int N, in
     g.si = (long)N * M;
     VortMarch vm;
     vm.tj = (N + TJ - 1) / TJ;
-    vm.tk = (M + 59) / 60;
-    // chunks of 16 planes (256^3: 8 planes 172 us, 32 planes 185); shorter
+    // 56 columns where they need no more tiles than 60: the rows of 448 bytes
+    // that each workgroup then writes end on 64-byte lines where M is a
+    // multiple of 8 (256^3: 169 -> 151 us; elsewhere equal)
+    vm.kw = (M + 55) / 56 == (M + 59) / 60 ? 56 : 60;
+    vm.tk = (M + vm.kw - 1) / vm.kw;
+    // chunks of 16 planes (256^3: 8 planes 180 us, 12 planes 162, 16 planes 151); shorter
     // ones, down to 4 planes, where those would not fill the chip once and the
     // shorter ones still run in one round (64^3: 4 planes 14 us, 16 planes 22)
     const long slots = 2L * device_cus();

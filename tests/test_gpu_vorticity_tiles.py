@@ -1,4 +1,4 @@
-"""The vorticity kernel's tiles on the GPU: 7 rows x 60 columns, chunks of 4
+"""The vorticity kernel's tiles on the GPU: 7 rows x 56 or 60 columns, chunks of 4
 to 16 planes by grid size, neighbours across rows from the previous step's
 planes.  Sizes lie on either side of each tile edge, with enough tiles for
 every chunk length; the kernel keeps the oracle's operand order in double, so
@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 # planes either side of one chunk of 4, rows of 7, columns of 60; (70, 150, 130)
 # takes chunks between 4 and 16 planes, (65, 222, 182) chunks of 16
-@pytest.mark.parametrize("shape", [(4, 7, 60), (5, 8, 61), (6, 6, 59), (7, 13, 62), (8, 14, 63), (9, 15, 122),
+@pytest.mark.parametrize("shape", [(4, 7, 60), (5, 8, 61), (6, 6, 59), (7, 13, 62), (8, 14, 63), (9, 15, 122), (4, 6, 56),
+                                   (5, 9, 112), (6, 10, 168), (4, 15, 240), (5, 7, 248),
                                    (17, 21, 64), (70, 150, 130), (65, 222, 182)])
 @pytest.mark.parametrize("precision", [2, 1, 3])
 def test_tile_edges(oracle, shape, precision):
