@@ -304,7 +304,7 @@ long long nlse_footprint_bytes(int dim, int N, int M, int L, int method, int pre
 /* ---- batched 2D API ----
  * nprob independent 2D problems (sizes N[p] x M[p], each with its own s, a,
  * h^2, k and potential V, one boundary code for all) advanced together: one
- * persistent kernel launch per fused group of RK4 stages walks the tiles of
+ * kernel launch per fused group of RK4 stages walks the tiles of
  * every problem.  precision: 2 = double (bit-identical to the reference CPU
  * integrator, problem by problem), 3 = single with a compensated hi + lo
  * state.  Problems are addressed by index p; states are double planes. */
@@ -328,10 +328,10 @@ int nlse_batch_diagnostics(nlse_batch *b, double *out);
  * (rows 8, 12, 16; default 16, a whole step per launch), 2 register strips (3..256-row segments, one
  * wave each); see nlse_set_kernel */
 int nlse_batch_set_kernel(nlse_batch *b, int kind, int rows);
-/* stages per launch, kernel kind, rows per tile, persistent grid */
+/* stages per launch, kernel kind, rows per tile, workgroups at most */
 int nlse_batch_get_config(const nlse_batch *b, int *fusion, int *kind, int *rows, int *grid);
 /* stages per launch (1, 2, 4), rows per tile (strip segment) of the current kernel family,
- * persistent grid (multiple of 8 workgroups) and hipGraph steps per replay
+ * workgroups at most (a multiple of 8; default: one per tile) and hipGraph steps per replay
  * (0 = off) */
 int nlse_batch_configure(nlse_batch *b, int stages_per_launch, int tile_rows, int grid,
                          int steps_per_graph);
@@ -344,7 +344,7 @@ int nlse_batch_autotune(nlse_batch *b, int steps, int *best_fusion, int *best_ti
 /* Groups of resident 2D solvers (no counterpart in the reference, which
  * solves one problem per call): the members (2D, one method and precision;
  * any sizes, parameters and boundaries) are advanced together by the batched
- * kernels, one persistent launch per RK4 step over the 16-row tiles of every
+ * kernels, one launch per RK4 step over the 16-row tiles of every
  * member, each in its own buffers.  Results are bit-identical to
  * stepping each member alone.  nlse_group_create waits for the members'
  * queued work; nlse_group_step enqueues on the group's own stream (returns

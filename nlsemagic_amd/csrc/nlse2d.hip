@@ -94,11 +94,8 @@ static hipError_t launch_strip(const StageArgs<T>& a, hipStream_t st)
 }
 
 // Row-sweep LDS tiles (nlse2d_rows.h): one workgroup per tile of TI rows.
-// At most 128 VGPRs (four waves per SIMD): the FP64 stage-3-4 tile would take
-// 132 and run three waves per SIMD, slower than with four waves and a few
-// registers spilled.
 template <typename T, int METHOD, int FIRST, int LAST, int TI, bool COMP, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void rows2d_kernel(const c2<T>* __restrict__ yin, const c2<T>* u,
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(rows_eu<T, METHOD>()))) void rows2d_kernel(const c2<T>* __restrict__ yin, const c2<T>* u,
                                                      c2<T>* __restrict__ acc, c2<T>* out, const T* __restrict__ V,
                                                      Coefs<T> c, Grid2 g, int BC, c2<T>* __restrict__ ulo)
 {
@@ -107,11 +104,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
     int ti, tj;
     if (!g.edge_first(blockIdx.x, ti, tj)) return;
     const int i0 = ti * TI - g.ioff, j0 = tj * W - g.joff;
-    if (rows_inner<METHOD, FIRST, LAST, TI>(i0, j0, g.N, g.M))
-        rows2d_tile<T, METHOD, FIRST, LAST, TI, COMP, true, NW>(sm, i0, j0, g.N, g.M, yin, u, acc, out, V, c, BC, ulo);
-    else
-        rows2d_tile<T, METHOD, FIRST, LAST, TI, COMP, false, NW>(sm, i0, j0, g.N, g.M, yin, u, acc, out, V, c, BC,
-                                                                 ulo);
+    // tiles of 8 rows on 16 waves are chosen where a launch is one round of tiles:
+    // no COLS case there (131 x 150 CD FP64 5.5 us, with it 5.65)
+    constexpr bool COLS = FIRST == 1 && LAST == 4 && !(TI == 8 && NW == 16);
+    rows2d_any<T, METHOD, FIRST, LAST, TI, COMP, NW, COLS>(sm, i0, j0, g.N, g.M, yin, u, acc, out, V, c, BC, ulo);
 }
 
 template <typename T, int METHOD, int FIRST, int LAST, int TI, int NW = rows_waves<METHOD, FIRST, LAST, TI>()>

@@ -1,5 +1,5 @@
 // nlse2d_batch.hip -- many independent 2D problems (uneven sizes, own s, a,
-// h, k and V each) advanced by ONE persistent launch per fused group of RK4
+// h, k and V each) advanced by ONE launch per fused group of RK4
 // stages.  Each workgroup walks the concatenated tile list of all problems;
 // the tile code is the single-problem one (nlse2d_tile.h, nlse2d_rows.h,
 // nlse2d_strip.h), so every problem's result is bit-identical to running it
@@ -10,7 +10,7 @@
 
 namespace nlse {
 
-// A persistent grid walks the concatenated tile list of all problems: block b
+// The grid walks the concatenated tile list of all problems: block b
 // works on XCD b mod 8, which owns a contiguous eighth of the list, so the
 // tiles of one problem (and their shared halos) stay in one L2.
 template <typename T, int METHOD, int TI, int FIRST, int LAST>
@@ -35,9 +35,13 @@ __global__ __launch_bounds__(256) void batch2d_kernel(const BatchProb2<T>* __res
     }
 }
 
-// the same walk over row-sweep tiles (tile width 64 - 2H per problem)
-template <typename T, int METHOD, int TI, int FIRST, int LAST, bool COMP, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void batch2d_rows_kernel(const BatchProb2<T>* __restrict__ probs,
+// the same walk over row-sweep tiles (tile width 64 - 2H per problem).  LOOP:
+// fewer workgroups than tiles (a grid the caller asked for).  One tile per
+// workgroup keeps nothing across tiles, so FP64 2SHOC spills 3 registers
+// instead of 17 and FP32c needs 79 instead of 93 (96 problems of sides 64-512,
+// per step: 239 -> 217 us and 167 -> 139).
+template <typename T, int METHOD, int TI, int FIRST, int LAST, bool COMP, int NW, bool LOOP>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(rows_eu<T, METHOD>()))) void batch2d_rows_kernel(const BatchProb2<T>* __restrict__ probs,
                                                            const int* __restrict__ tile_prob, int ntiles,
                                                            int r_yin, int r_u, int r_out)
 {
@@ -47,19 +51,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
     const int per = (ntiles + 7) >> 3;
     for (int i = blockIdx.x >> 3; i < per; i += nper) {
         const int t = xcd * per + i;
-        if (t >= ntiles) break;
+        if (t >= ntiles) return;
         const BatchProb2<T>& P = probs[tile_prob[t]];
         const int lt = t - P.tile0;
         const int ti = lt / P.tiles_j, tj = lt - ti * P.tiles_j;
-        const int i0 = ti * TI - P.ioff, j0 = tj * W - P.joff;
-        c2<T>* lo = COMP ? P.ulo : nullptr;
-        if (rows_inner<METHOD, FIRST, LAST, TI>(i0, j0, P.N, P.M))
-            rows2d_tile<T, METHOD, FIRST, LAST, TI, COMP, true, NW>(sm, i0, j0, P.N, P.M, P.buf[r_yin], P.buf[r_u],
-                                                                    P.acc, P.buf[r_out], P.V, P.c, P.BC, lo);
-        else
-            rows2d_tile<T, METHOD, FIRST, LAST, TI, COMP, false, NW>(sm, i0, j0, P.N, P.M, P.buf[r_yin],
-                                                                     P.buf[r_u], P.acc, P.buf[r_out], P.V, P.c,
-                                                                     P.BC, lo);
+        rows2d_any<T, METHOD, FIRST, LAST, TI, COMP, NW, FIRST == 1 && LAST == 4>(sm, ti * TI - P.ioff, tj * W - P.joff, P.N, P.M,
+                                                               P.buf[r_yin], P.buf[r_u], P.acc, P.buf[r_out], P.V,
+                                                               P.c, P.BC, COMP ? P.ulo : nullptr);
+        if (!LOOP) return;
         __syncthreads();  // the next tile reuses the LDS
     }
 }
@@ -103,20 +102,27 @@ static hipError_t launch_b_strips(const BatchArgs<T>& a, hipStream_t st)
     return hipGetLastError();
 }
 
-template <typename T, int METHOD, int TI, int FIRST, int LAST>
-static hipError_t launch_b_rows(const BatchArgs<T>& a, hipStream_t st)
+template <typename T, int METHOD, int TI, int FIRST, int LAST, bool COMP>
+static hipError_t launch_b_rows_c(const BatchArgs<T>& a, hipStream_t st)
 {
     constexpr int NW = rows_waves<METHOD, FIRST, LAST, TI>();
-    if constexpr (std::is_same<T, float>::value && LAST == 4) {
-        if (a.comp) {
-            hipLaunchKernelGGL((batch2d_rows_kernel<T, METHOD, TI, FIRST, LAST, true, NW>), dim3(a.grid),
+    if constexpr (FIRST == 1 && LAST == 4)  // the default split; the others keep the loop
+        if (a.grid >= a.ntiles) {
+            hipLaunchKernelGGL((batch2d_rows_kernel<T, METHOD, TI, FIRST, LAST, COMP, NW, false>), dim3(a.grid),
                                dim3(NW * 64), 0, st, a.probs, a.tile_prob, a.ntiles, a.r_yin, a.r_u, a.r_out);
             return hipGetLastError();
         }
-    }
-    hipLaunchKernelGGL((batch2d_rows_kernel<T, METHOD, TI, FIRST, LAST, false, NW>), dim3(a.grid), dim3(NW * 64), 0,
-                       st, a.probs, a.tile_prob, a.ntiles, a.r_yin, a.r_u, a.r_out);
+    hipLaunchKernelGGL((batch2d_rows_kernel<T, METHOD, TI, FIRST, LAST, COMP, NW, true>), dim3(a.grid), dim3(NW * 64),
+                       0, st, a.probs, a.tile_prob, a.ntiles, a.r_yin, a.r_u, a.r_out);
     return hipGetLastError();
+}
+
+template <typename T, int METHOD, int TI, int FIRST, int LAST>
+static hipError_t launch_b_rows(const BatchArgs<T>& a, hipStream_t st)
+{
+    if constexpr (std::is_same<T, float>::value && LAST == 4)
+        if (a.comp) return launch_b_rows_c<T, METHOD, TI, FIRST, LAST, true>(a, st);
+    return launch_b_rows_c<T, METHOD, TI, FIRST, LAST, false>(a, st);
 }
 
 template <typename T, int METHOD, int TI, int FIRST, int LAST>

@@ -64,6 +64,13 @@ constexpr int rows_waves()
     return RowsCfg<METHOD, FIRST, LAST, TI>::TE > 16 ? 8 : 4;
 }
 
+// waves per SIMD that the registers are held to.  Workgroups of 8 waves come
+// two to a SIMD, so 5 waves are worth 4.  FP32 2SHOC: at most 80 registers and
+// 6 waves, where the batch kernel would take 81 to 93 (96 problems FP32c 146 ->
+// 127 us per step).  FP64 2SHOC: 128 and 4; the stage-3-4 tile would take 132,
+// and three waves are slower than four with a few registers spilled.
+template <typename T, int METHOD> constexpr int rows_eu() { return sizeof(T) == 4 && METHOD == 2 ? 6 : 4; }
+
 template <int METHOD, int FIRST, int LAST, int TI, int NW>
 struct RowsCfg {
     static constexpr int R = (METHOD == 2) ? 2 : 1;
@@ -91,17 +98,24 @@ struct RowsLds {
 
 // Tile with owned rows [i0, i0 + TI) and columns [j0, j0 + W) of an N x M
 // problem (the block may overhang the grid by one row/column at the start
-// and by any amount at the end).  Buffers as in fused2d_tile.  INNER: the
-// extended tile lies inside the grid and holds no boundary row or column
-// (rows_inner()), so every range below is a compile-time constant.
+// and by any amount at the end).  Buffers as in fused2d_tile.  RIN: every
+// row whose D or F is evaluated is an interior row of the grid, so every row
+// range below is a compile-time constant; CIN: the extended tile's columns are
+// interior.
 template <int METHOD, int FIRST, int LAST, int TI>
-__device__ __forceinline__ bool rows_inner(int i0, int j0, int N, int M)
+__device__ __forceinline__ bool rows_inside(int i0, int N)
 {
     using Cfg = RowsCfg<METHOD, FIRST, LAST, TI>;
-    return i0 - Cfg::H >= 0 && i0 - Cfg::H + Cfg::TE <= N && j0 - Cfg::H >= 1 && j0 - Cfg::H + 64 <= M - 1;
+    return i0 - Cfg::H >= 0 && i0 - Cfg::H + Cfg::TE <= N;
+}
+template <int METHOD, int FIRST, int LAST, int TI>
+__device__ __forceinline__ bool cols_inside(int j0, int M)
+{
+    using Cfg = RowsCfg<METHOD, FIRST, LAST, TI>;
+    return j0 - Cfg::H >= 1 && j0 - Cfg::H + 64 <= M - 1;
 }
 
-template <typename T, int METHOD, int FIRST, int LAST, int TI, bool COMP, bool INNER, int NW = 4>
+template <typename T, int METHOD, int FIRST, int LAST, int TI, bool COMP, bool RIN, bool CIN, int NW = 4>
 __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>& sm, int i0, int j0, int N, int M,
                                             const c2<T>* __restrict__ yin, const c2<T>* u, c2<T>* __restrict__ acc,
                                             c2<T>* out, const T* __restrict__ V, const Coefs<T>& c, int BC,
@@ -114,22 +128,22 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     __builtin_assume(w >= 0 && w < NW);
     const int j = j0 - H + lane;
-    const bool jin = INNER || (j >= 0 && j < M);
+    const bool jin = CIN || (j >= 0 && j < M);
     const bool own = jin && lane >= H && lane < H + W;
-    const int jc = INNER ? j : (j < 0 ? 0 : (j >= M ? M - 1 : j));
+    const int jc = CIN ? j : (j < 0 ? 0 : (j >= M ? M - 1 : j));
     const bool colL = (j == 0), colR = (j == M - 1);
     const int lL = H - j0, lR = M - 1 - j0 + H;
-    const bool colbc = !INNER && ((lL >= 0 && lL < 64) || (lR >= 0 && lR < 64));
+    const bool colbc = !CIN && ((lL >= 0 && lL < 64) || (lR >= 0 && lR < 64));
     const int g0 = i0 - H;  // grid row of extended row 0
     // extended rows inside the grid: [eg0, eg1)
-    const int eg0 = INNER ? 0 : -g0, eg1 = INNER ? TE : N - g0;
+    const int eg0 = RIN ? 0 : -g0, eg1 = RIN ? TE : N - g0;
     const bool msd = (BC == BC_MSD);
-    const bool top = !INNER && msd && eg0 >= 0 && eg0 < TE, bot = !INNER && msd && eg1 - 1 >= 0 && eg1 - 1 < TE;
+    const bool top = !RIN && msd && eg0 >= 0 && eg0 < TE, bot = !RIN && msd && eg1 - 1 >= 0 && eg1 - 1 < TE;
     // MSD columns 0 / M-1 in this tile (uniform over the workgroup): their D
     // comes from the column pass after each D phase
-    const bool colmsd = !INNER && msd && colbc;
+    const bool colmsd = !CIN && msd && colbc;
     // a D/F row at grid row g is interior (the reference's full stencil)
-    auto interior = [&](int g) { return INNER || (g > 0 && g < N - 1); };
+    auto interior = [&](int g) { return RIN || (g > 0 && g < N - 1); };
     const c2<T> z = mk<T>(0, 0);
 
     auto sy = [&](int e, int dl) -> c2<T> { return sm.y[1 + e * 64 + lane + dl]; };
@@ -154,7 +168,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
     // read clamped rows: values no owned point uses)
     auto rowp = [&](int e) -> long {
         const int g = g0 + e;
-        const int gc = INNER ? g : (g < 0 ? 0 : (g >= N ? N - 1 : g));
+        const int gc = RIN ? g : (g < 0 ? 0 : (g >= N ? N - 1 : g));
         return (long)gc * M + jc;
     };
 #pragma unroll
@@ -187,14 +201,16 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
     }
     __syncthreads();
 
-#pragma unroll
+    // "unroll 4" unrolls it whole, like a bare unroll, but later in the
+    // compilation, which leaves fewer registers spilled
+#pragma unroll 4
     for (int q = 0; q < NF; ++q) {
         const int QS = FIRST + q;
         // F rows and D rows of this stage
-        const int flo = INNER ? (q + 1) * R : max((q + 1) * R, eg0);
-        const int fhi = INNER ? TE - (q + 1) * R : min(TE - (q + 1) * R, eg1);
-        const int dlo = INNER ? (q + 1) * R - 1 : max((q + 1) * R - 1, eg0);
-        const int dhi = INNER ? TE - (q + 1) * R + 1 : min(TE - (q + 1) * R + 1, eg1);
+        const int flo = RIN ? (q + 1) * R : max((q + 1) * R, eg0);
+        const int fhi = RIN ? TE - (q + 1) * R : min(TE - (q + 1) * R, eg1);
+        const int dlo = RIN ? (q + 1) * R - 1 : max((q + 1) * R - 1, eg0);
+        const int dhi = RIN ? TE - (q + 1) * R + 1 : min(TE - (q + 1) * R + 1, eg1);
         c2<T> ypart[RW];  // MSD boundary rows: the partner row's Y, read before the Y rows change
 #pragma unroll
         for (int k = 0; k < RW; ++k) ypart[k] = z;
@@ -359,6 +375,30 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
         }
         if (q < NF - 1) __syncthreads();  // the next stage's input rows are in LDS
     }
+}
+
+// The tile by where it lies: inside the grid, on its first or last columns only
+// (COLS), or on the first or last rows.  The general code takes half as long
+// again even where no boundary is near (1024^2 with it throughout: 2SHOC FP64
+// 30.4 -> 37.9 us per step, CD FP32 8.6 -> 13.1), and in problems of a few
+// hundred points a side a third of the tiles lie on the edge columns.  Per
+// step, without -> with COLS: 96 problems of sides 64-512 2SHOC FP64 217 ->
+// 200 us, FP32c 139 -> 127, CD FP32c 63 -> 53; 8 problems 2SHOC FP64 31.9 ->
+// 27.0; 517 x 389 2SHOC FP64 16.3 -> 15.6.  One more case for the first and
+// last rows gained nothing.
+template <typename T, int METHOD, int FIRST, int LAST, int TI, bool COMP, int NW, bool COLS>
+__device__ __forceinline__ void rows2d_any(RowsLds<T, METHOD, FIRST, LAST, TI>& sm, int i0, int j0, int N, int M,
+                                           const c2<T>* __restrict__ yin, const c2<T>* u, c2<T>* __restrict__ acc,
+                                           c2<T>* out, const T* __restrict__ V, const Coefs<T>& c, int BC,
+                                           c2<T>* __restrict__ ulo)
+{
+    const bool rin = rows_inside<METHOD, FIRST, LAST, TI>(i0, N), cin = cols_inside<METHOD, FIRST, LAST, TI>(j0, M);
+    if (rin && cin)
+        rows2d_tile<T, METHOD, FIRST, LAST, TI, COMP, true, true, NW>(sm, i0, j0, N, M, yin, u, acc, out, V, c, BC, ulo);
+    else if (COLS && rin)
+        rows2d_tile<T, METHOD, FIRST, LAST, TI, COMP, true, false, NW>(sm, i0, j0, N, M, yin, u, acc, out, V, c, BC, ulo);
+    else
+        rows2d_tile<T, METHOD, FIRST, LAST, TI, COMP, false, false, NW>(sm, i0, j0, N, M, yin, u, acc, out, V, c, BC, ulo);
 }
 
 }  // namespace nlse

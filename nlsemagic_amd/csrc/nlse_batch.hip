@@ -1,6 +1,6 @@
 // nlse_batch.hip -- C ABI of the batched 2D integrator (include/nlsemagic_hip.h,
 // nlse_batch_*): many independent 2D problems of uneven size, each with its
-// own s, a, h^2, k and potential, advanced together by one persistent launch
+// own s, a, h^2, k and potential, advanced together by one launch
 // per fused group of RK4 stages.  The state of every problem stays resident;
 // problem p's fields live at element offset off[p] of shared buffers.
 #include <algorithm>
@@ -36,6 +36,9 @@ struct nlse_batch {
 };
 
 namespace {
+
+// workgroups per launch: a tile each (launches take no more than they need)
+constexpr int GRID_ALL = 1 << 20;
 
 int fail(int code, const std::string& msg) { return set_error(code, msg); }
 
@@ -255,18 +258,18 @@ int nlse_batch_create(nlse_batch** out, int nprob, const int* N, const int* M, c
         o += (long)N[p] * M[p];
     }
     b->ntot = ntot;
-    // a whole RK4 step per launch on row-sweep tiles of 16 rows, and a grid
-    // of several tiles' worth of workgroups per CU, so that the hardware
-    // evens out the unequal tiles.  Per step, pairs of stages on 8-row tiles
-    // with 4 workgroups per CU -> this: 96 problems of sides 64-512 2SHOC FP64
-    // 268 -> 220 us, FP32c 193 -> 159, CD FP64 203 -> 94, FP32c 138 -> 66; 8
-    // problems 2SHOC FP64 36 -> 32, FP32c 29 -> 25.
+    // a whole RK4 step per launch on row-sweep tiles of 16 rows, and a
+    // workgroup for every tile, so that the hardware evens out the unequal
+    // tiles.  Per step, pairs of stages on 8-row tiles with 4 workgroups per CU
+    // -> this: 96 problems of sides 64-512 2SHOC FP64 268 -> 200 us, FP32c 193
+    // -> 127, CD FP64 203 -> 94, FP32c 138 -> 53; 8 problems 2SHOC FP64 36 ->
+    // 27, FP32c 29 -> 19.  (Of that, by one tile per workgroup instead of a
+    // loop over tiles, which keeps registers: 239 -> 217 us 2SHOC FP64, 167 ->
+    // 139 FP32c.)
     b->fuse = 4;
     b->kern = KERNEL_ROWS;
     b->tile = 16;
-    int cus = 256;
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0);
-    b->grid = 8 * ((cus * 32 + 7) / 8);
+    b->grid = GRID_ALL;
     const size_t eb = (precision == 2 ? 16 : 8) * (size_t)ntot;
     void** bufs[5] = {&b->U, &b->Y0, &b->Y1, &b->acc, &b->V};
     for (int i = 0; i < 5; ++i)
@@ -465,7 +468,7 @@ int nlse_batch_autotune(nlse_batch* b, int steps, int* best_fusion, int* best_ti
     if (saved_lo) HIPCHK(hipMemcpyAsync(saved_lo, b->Ulo, eb, hipMemcpyDeviceToDevice, b->stream));
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0);
-    const int fz[3] = {1, 2, 4}, occ[3] = {2, 4, 8};
+    const int fz[3] = {1, 2, 4}, gr[3] = {8 * ((cus * 4 + 7) / 8), 8 * ((cus * 8 + 7) / 8), GRID_ALL};
     // rows per tile (strips: per segment) of each kernel family
     const int tl[3][3] = {{8, 16, 32}, {8, 12, 16}, {16, 32, 64}};
     const int gsave = b->gsteps;
@@ -477,7 +480,7 @@ int nlse_batch_autotune(nlse_batch* b, int steps, int* best_fusion, int* best_ti
             for (int y = 0; y < 3 && rc == NLSE_OK; ++y)
                 for (int z = 0; z < 3 && rc == NLSE_OK; ++z) {
                     rc = nlse_batch_set_kernel(b, kind, tl[kind][y]);
-                    if (rc == NLSE_OK) rc = nlse_batch_configure(b, fz[x], tl[kind][y], 8 * ((cus * occ[z] + 7) / 8), 0);
+                    if (rc == NLSE_OK) rc = nlse_batch_configure(b, fz[x], tl[kind][y], gr[z], 0);
                     if (rc == NLSE_OK) rc = enqueue_steps(b, 1);
                     double ms = 0;
                     if (rc == NLSE_OK) rc = nlse_batch_step_timed(b, steps, &ms);

@@ -1590,8 +1590,8 @@ int NLSE3D_VORTICITY_HIP(const double* Ur, const double* Ui, double lh2, double 
 // ---- groups of resident 2D solvers advanced by shared launches
 //
 // The solvers keep their own buffers; a problem table points the batched 2D
-// kernels (nlse2d_batch.hip) at them, so one persistent launch per fused pair
-// of RK4 stages walks the tiles of every member.  The tile code and each
+// kernels (nlse2d_batch.hip) at them, so one launch per RK4 step
+// walks the tiles of every member.  The tile code and each
 // member's coefficients are the solver's own: a member's result is bit for
 // bit the result of stepping it alone.
 
@@ -1600,7 +1600,7 @@ struct nlse_group {
     int method, prec;
     void* probs;     // device BatchProb2<T>[n]
     int* tile_prob;  // device: member of each tile
-    int ntiles, grid;
+    int ntiles;
     int parity;      // fused steps taken mod 2: buffers 0 and 2 of the table have swapped roles
     hipStream_t stream;
 };
@@ -1664,7 +1664,7 @@ int group_launch_t(nlse_group* g, int first, int last, int r_yin, int r_out)
     a.first = first;
     a.last = last;
     a.tile = GROUP_ROWS;
-    a.grid = std::min(g->grid, 8 * ((g->ntiles + 7) / 8));
+    a.grid = 8 * ((g->ntiles + 7) / 8);  // a workgroup per tile, as a batch's default
     a.kernel = KERNEL_ROWS;
     const hipError_t e = launch_batch2d<T>(a, g->stream);
     if (e != hipSuccess) return fail(NLSE_EHIP, std::string("group launch: ") + hipGetErrorString(e));
@@ -1708,9 +1708,6 @@ int nlse_group_create(nlse_group** out, nlse_solver* const* members, int n)
     g->tile_prob = nullptr;
     g->parity = 0;
     g->stream = nullptr;
-    int cus = 256;
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0);
-    g->grid = 8 * ((cus * 32 + 7) / 8);  // as a batch's (nlse_batch_create)
     // the members' queued work finishes before the group touches their buffers
     for (nlse_solver* h : g->mem)
         if (hipStreamSynchronize(h->stream) != hipSuccess) {

@@ -65,7 +65,7 @@ struct BatchProb2 {
     Coefs<T> c;
 };
 
-// One persistent launch of RK4 stages first..last over every tile of a batch
+// One launch of RK4 stages first..last over every tile of a batch
 // of 2D problems (`tile` = rows per tile, or per strip segment for
 // KERNEL_STRIPS; `grid` workgroups, a multiple of 8): stage input
 // buf[r_yin], U = buf[r_u], output buf[r_out] of every problem.

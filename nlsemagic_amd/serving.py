@@ -16,7 +16,7 @@ compensated FP32, step count, initial state and potential).  The server:
   to drain;
 - batches the 2D requests: the active 2D requests of one method and
   precision take their chunks together as a group (nlse_group_*), one
-  persistent launch per pair of RK4 stages over the tiles of all of them
+  launch per RK4 step over the tiles of all of them
   (each in its own buffers), the chunk being the smallest number of steps
   any of them has left (at most ``chunk_steps``); a 2D request that is ready
   while others of its kind are still working waits for them, so a request

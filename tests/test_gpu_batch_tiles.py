@@ -1,0 +1,45 @@
+"""Batches on the GPU with a workgroup per tile and with fewer, over sizes on
+either side of the row-sweep tile's edges (16 rows; 48 columns for 2SHOC, 56
+for CD), so that tiles inside the grid, on its edge columns only and on its
+first or last rows all occur: every problem equals the same problem stepped
+alone by the LDS-tile kernels, bit for bit (double also against the oracle)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import bits_equal
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(15, 47), (16, 48), (17, 49), (33, 97), (49, 56), (50, 57), (81, 113), (97, 145), (161, 168), (65, 170)]
+
+
+@pytest.mark.parametrize("BC", [1, 2, 3])
+@pytest.mark.parametrize("method,precision", [(1, 2), (2, 2), (1, 3), (2, 3)])
+@pytest.mark.parametrize("grid", [None, 8])
+def test_batch_tiles(oracle, method, precision, BC, grid):
+    import nlsemagic_amd as nm
+    print("CASE batch tiles", method, precision, BC, grid, flush=True)
+    rng = np.random.default_rng(7)
+    n = len(SHAPES)
+    s, a = [(-1.0) ** i for i in range(n)], [0.5 + 0.05 * i for i in range(n)]
+    h2, k = [0.04] * n, [0.003] * n
+    U = [1 + 0.2 * rng.uniform(-1, 1, sh) + 0.2j * rng.uniform(-1, 1, sh) for sh in SHAPES]
+    V = [0.3 * rng.uniform(-1, 1, sh) for sh in SHAPES]
+    B = nm.Batch(SHAPES, s, a, h2, k, method=method, precision=precision, BC=BC)
+    if grid:
+        B.configure(4, 16, grid, 0)
+    for i in range(n):
+        B.set_state(i, U[i], V[i])
+    B.step(3)
+    for i in range(n):
+        S = nm.Solver(SHAPES[i], method, precision, BC, s[i], a[i], h2[i], k[i])
+        S.set_kernel(0, 8)
+        S.set_state(U[i], V[i])
+        S.step(3)
+        assert bits_equal(B.state(i), S.state()), SHAPES[i]
+        S.close()
+        if precision == 2:
+            assert bits_equal(B.state(i), oracle.take_steps(U[i], V[i], s[i], a[i], h2[i], BC, 3, k[i], method)), SHAPES[i]
+    B.close()
