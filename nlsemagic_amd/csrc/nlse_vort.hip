@@ -35,7 +35,7 @@
 // 159 us at the rate of a large copy).  Per call, 16 rows on 16 waves with a
 // branch per difference and loads widened at once -> this: 256^3 FP64 244 ->
 // 151 us, FP32 275 -> 149, FP32c 333 -> 158; 201 x 180 x 190 FP64 150 -> 99;
-// 64^3 FP64 68 -> 14.
+// 64^3 FP64 68 -> 14; 256^3 of four vortex rings 258 -> 191.
 #include "nlse2d_strip.h"
 #include "nlse_host.h"
 
