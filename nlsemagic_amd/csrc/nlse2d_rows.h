@@ -20,7 +20,9 @@
 //     lane shifts FP64 15.8 -> 16.3 us, FP32 equal);
 //   - per stage: D phase, barrier, F phase (each row's F and RK4 update at
 //     once, the new Y in the row's registers), barrier, new Y rows written
-//     to LDS, barrier; the last stage writes its rows to HBM.
+//     to LDS, barrier (rows_early(): the corner terms in the D phase, the new Y
+//     to LDS in the F phase, one barrier less); the last stage writes its rows
+//     to HBM.
 // MSD boundary rows take their partner row's D/F from LDS after the barrier
 // that completes it (D: one extra barrier, only in tiles holding row 0 or
 // N-1).  MSD boundary columns take the partner lane's F by DPP; their D is
@@ -96,6 +98,19 @@ struct RowsLds {
     T bv[Cfg::TE][4];
 };
 
+// Whether the D phase also forms the corner terms of F (4 registers per row).
+// The F phase then reads no Y but the row's own, so each row's new Y goes to LDS
+// at once and a stage has two barriers instead of three.  FP64 whole steps on 8
+// waves, per step: 1024^2 30.9 -> 28.8 us (MSD 31.9 -> 30.0), 700^2 18.7 -> 17.2,
+// 512^2 10.8 -> 10.5, 96 problems of sides 64-512 204 -> 194.  On 16 waves, where
+// a launch is one round of tiles, MSD loses (131 x 150 10.5 -> 10.8), and single
+// precision gains nothing at 1024^2 and loses up to 3 % below.  The row's own D
+// held as well: 47-56 registers spilled, 96 problems 210 us.
+template <typename T, int METHOD, int FIRST, int LAST, int NW> constexpr bool rows_early()
+{
+    return METHOD == 2 && sizeof(T) == 8 && FIRST == 1 && LAST == 4 && NW == 8;
+}
+
 // Tile with owned rows [i0, i0 + TI) and columns [j0, j0 + W) of an N x M
 // problem (the block may overhang the grid by one row/column at the start
 // and by any amount at the end).  Buffers as in fused2d_tile.  RIN: every
@@ -157,6 +172,13 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
         return colL ? p : (colR ? m : v);
     };
 
+    // the 2SHOC stencil's corner term of row e
+    auto corners = [&](int e, c2<T> yx) -> c2<T> {
+        const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
+        return mk<T>(aa.x + ab.x - 4 * yx.x + ba.x + bb.x, aa.y + ab.y - 4 * yx.y + ba.y + bb.y);
+    };
+    constexpr bool EARLY = rows_early<T, METHOD, FIRST, LAST, NW>();
+
     // rows of this wave: e = 4k + w; everything about row e stays in slot k
     c2<T> Yc[RW], Uc[RW], Ac[RW], Lc[RW];
     T Vc[RW];
@@ -214,6 +236,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
         c2<T> ypart[RW];  // MSD boundary rows: the partner row's Y, read before the Y rows change
 #pragma unroll
         for (int k = 0; k < RW; ++k) ypart[k] = z;
+        c2<T> Gc[RW];  // EARLY: the corner terms of F, formed in the D phase
         if constexpr (METHOD == 2) {
 #pragma unroll
             for (int k = 0; k < RW; ++k) {
@@ -221,6 +244,14 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 if (e < dlo || e >= dhi) continue;
                 const int g = g0 + e;
                 const c2<T> yx = Yc[k];
+                if (EARLY && e >= flo && e < fhi) {
+                    if (interior(g)) {
+                        Gc[k] = corners(e, yx);
+                        pin_here<T>(Gc[k]);
+                    } else if (msd) {
+                        ypart[k] = sy(g == 0 ? e + 1 : e - 1, 0);
+                    }
+                }
                 const T vx = Vc[k];
                 c2<T> dd = z;
                 if (interior(g)) {
@@ -325,11 +356,13 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 if constexpr (METHOD == 2) {
                     const c2<T> dc = sd(e, 0), da = sd(e + 1, 0), db = sd(e - 1, 0);
                     const c2<T> dl = lane_shift2<DPP_NEXT, T>(dc), dr = lane_shift2<DPP_PREV, T>(dc);
-                    const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
+                    c2<T> gc;
+                    if constexpr (EARLY) gc = Gc[k];
+                    else gc = corners(e, yx);
                     ff = mk<T>(-c.a * dc.y + c.a1_12 * (da.y + db.y + dl.y + dr.y)
-                                   - c.a1_6h2 * (aa.y + ab.y - 4 * yx.y + ba.y + bb.y) - n * yx.y,
+                                   - c.a1_6h2 * gc.y - n * yx.y,
                                c.a * dc.x - c.a1_12 * (da.x + db.x + dl.x + dr.x)
-                                   + c.a1_6h2 * (aa.x + ab.x - 4 * yx.x + ba.x + bb.x) + n * yx.x);
+                                   + c.a1_6h2 * gc.x + n * yx.x);
                 } else {
                     const c2<T> a = sy(e + 1, 0), b = sy(e - 1, 0);
                     const c2<T> l = sy(e, 1), rt = sy(e, -1);
@@ -347,14 +380,16 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
             } else if (BC == BC_LAP0) {
                 ff = lap0_f<T>(yx, vx, c.s);
             } else if (msd) {  // row 0 or N-1: F after the barrier
-                ypart[k] = sy(g == 0 ? e + 1 : e - 1, 0);
+                if (!EARLY) ypart[k] = sy(g == 0 ? e + 1 : e - 1, 0);
                 continue;
             }
             epilogue(k, e, ff);
+            if (EARLY && q < NF - 1) sm.y[1 + e * 64 + lane] = Yc[k];
             ROWS_SCHED_FENCE();
         }
         // every read of this stage's Y and D rows is done (after the last
-        // stage only the MSD boundary rows below still read LDS)
+        // stage only the MSD boundary rows below still read LDS; EARLY: the new Y
+        // rows are in LDS, but for rows 0 and N-1)
         if (q < NF - 1 || top || bot) __syncthreads();
         if (top || bot) {
 #pragma unroll
@@ -362,18 +397,19 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 const int e = NW * k + w;
                 if (e < flo || e >= fhi) continue;
                 const int g = g0 + e;
-                if (g == 0) epilogue(k, e, msd_f<T>(colq(sm.y[1 + lane]), colq(ypart[k]), Yc[k]));
-                else if (g == N - 1) epilogue(k, e, msd_f<T>(colq(sm.y[1 + (TE - 1) * 64 + lane]), colq(ypart[k]), Yc[k]));
+                if (g != 0 && g != N - 1) continue;
+                epilogue(k, e, msd_f<T>(colq(sm.y[1 + (g == 0 ? 0 : TE - 1) * 64 + lane]), colq(ypart[k]), Yc[k]));
+                if (EARLY && q < NF - 1) sm.y[1 + e * 64 + lane] = Yc[k];
             }
         }
-        if (q < NF - 1) {
+        if (!EARLY && q < NF - 1) {
 #pragma unroll
             for (int k = 0; k < RW; ++k) {
                 const int e = NW * k + w;
                 if (e >= flo && e < fhi) sm.y[1 + e * 64 + lane] = Yc[k];
             }
         }
-        if (q < NF - 1) __syncthreads();  // the next stage's input rows are in LDS
+        if (q < NF - 1 && (!EARLY || top || bot)) __syncthreads();  // the next stage's input rows are in LDS
     }
 }
 
