@@ -172,11 +172,6 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
         return colL ? p : (colR ? m : v);
     };
 
-    // the 2SHOC stencil's corner term of row e
-    auto corners = [&](int e, c2<T> yx) -> c2<T> {
-        const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
-        return mk<T>(aa.x + ab.x - 4 * yx.x + ba.x + bb.x, aa.y + ab.y - 4 * yx.y + ba.y + bb.y);
-    };
     constexpr bool EARLY = rows_early<T, METHOD, FIRST, LAST, NW>();
 
     // rows of this wave: e = 4k + w; everything about row e stays in slot k
@@ -246,7 +241,8 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 const c2<T> yx = Yc[k];
                 if (EARLY && e >= flo && e < fhi) {
                     if (interior(g)) {
-                        Gc[k] = corners(e, yx);
+                        const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
+                        Gc[k] = mk<T>(aa.x + ab.x - 4 * yx.x + ba.x + bb.x, aa.y + ab.y - 4 * yx.y + ba.y + bb.y);
                         pin_here<T>(Gc[k]);
                     } else if (msd) {
                         ypart[k] = sy(g == 0 ? e + 1 : e - 1, 0);
@@ -356,13 +352,17 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 if constexpr (METHOD == 2) {
                     const c2<T> dc = sd(e, 0), da = sd(e + 1, 0), db = sd(e - 1, 0);
                     const c2<T> dl = lane_shift2<DPP_NEXT, T>(dc), dr = lane_shift2<DPP_PREV, T>(dc);
-                    c2<T> gc;
-                    if constexpr (EARLY) gc = Gc[k];
-                    else gc = corners(e, yx);
-                    ff = mk<T>(-c.a * dc.y + c.a1_12 * (da.y + db.y + dl.y + dr.y)
-                                   - c.a1_6h2 * gc.y - n * yx.y,
-                               c.a * dc.x - c.a1_12 * (da.x + db.x + dl.x + dr.x)
-                                   + c.a1_6h2 * gc.x + n * yx.x);
+                    if constexpr (EARLY) {
+                        const c2<T> gc = Gc[k];
+                        ff = mk<T>(-c.a * dc.y + c.a1_12 * (da.y + db.y + dl.y + dr.y) - c.a1_6h2 * gc.y - n * yx.y,
+                                   c.a * dc.x - c.a1_12 * (da.x + db.x + dl.x + dr.x) + c.a1_6h2 * gc.x + n * yx.x);
+                    } else {
+                        const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
+                        ff = mk<T>(-c.a * dc.y + c.a1_12 * (da.y + db.y + dl.y + dr.y)
+                                       - c.a1_6h2 * (aa.y + ab.y - 4 * yx.y + ba.y + bb.y) - n * yx.y,
+                                   c.a * dc.x - c.a1_12 * (da.x + db.x + dl.x + dr.x)
+                                       + c.a1_6h2 * (aa.x + ab.x - 4 * yx.x + ba.x + bb.x) + n * yx.x);
+                    }
                 } else {
                     const c2<T> a = sy(e + 1, 0), b = sy(e - 1, 0);
                     const c2<T> l = sy(e, 1), rt = sy(e, -1);
@@ -397,9 +397,9 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 const int e = NW * k + w;
                 if (e < flo || e >= fhi) continue;
                 const int g = g0 + e;
-                if (g != 0 && g != N - 1) continue;
-                epilogue(k, e, msd_f<T>(colq(sm.y[1 + (g == 0 ? 0 : TE - 1) * 64 + lane]), colq(ypart[k]), Yc[k]));
-                if (EARLY && q < NF - 1) sm.y[1 + e * 64 + lane] = Yc[k];
+                if (g == 0) epilogue(k, e, msd_f<T>(colq(sm.y[1 + lane]), colq(ypart[k]), Yc[k]));
+                else if (g == N - 1) epilogue(k, e, msd_f<T>(colq(sm.y[1 + (TE - 1) * 64 + lane]), colq(ypart[k]), Yc[k]));
+                if (EARLY && q < NF - 1 && (g == 0 || g == N - 1)) sm.y[1 + e * 64 + lane] = Yc[k];
             }
         }
         if (!EARLY && q < NF - 1) {
