@@ -37,8 +37,8 @@ __global__ __launch_bounds__(256) void batch2d_kernel(const BatchProb2<T>* __res
 
 // the same walk over row-sweep tiles (tile width 64 - 2H per problem).  LOOP:
 // fewer workgroups than tiles (a grid the caller asked for).  One tile per
-// workgroup keeps nothing across tiles, so FP64 2SHOC spills 3 registers
-// instead of 17 and FP32c needs 79 instead of 93 (96 problems of sides 64-512,
+// workgroup keeps nothing across tiles, so FP64 2SHOC spills 2 registers
+// instead of 14 and FP32c needs 79 instead of 93 (96 problems of sides 64-512,
 // per step: 239 -> 217 us and 167 -> 139).
 template <typename T, int METHOD, int TI, int FIRST, int LAST, bool COMP, int NW, bool LOOP>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(rows_eu<T, METHOD>()))) void batch2d_rows_kernel(const BatchProb2<T>* __restrict__ probs,

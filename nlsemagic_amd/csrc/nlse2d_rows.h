@@ -16,7 +16,7 @@
 //     i +- 1 from an LDS copy of D.  A row's own j +- 1 neighbours: 2SHOC shifts
 //     lanes (DPP), which takes 4 of its 15 LDS accesses per row and stage away
 //     (1024^2 per step: FP32 19.2 -> 18.1 us, FP32c 20.8 -> 20.0, FP64 30.3 ->
-//     30.0, which then needs no spill); CD reads lane +- 1 of the LDS copy (with
+//     30.0); CD reads lane +- 1 of the LDS copy (with
 //     lane shifts FP64 15.8 -> 16.3 us, FP32 equal);
 //   - per stage: D phase, barrier, F phase (each row's F and RK4 update at
 //     once, the new Y in the row's registers), barrier, new Y rows written
