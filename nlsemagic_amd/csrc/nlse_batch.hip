@@ -271,9 +271,10 @@ int nlse_batch_create(nlse_batch** out, int nprob, const int* N, const int* M, c
     b->tile = 16;
     b->grid = GRID_ALL;
     const size_t eb = (precision == 2 ? 16 : 8) * (size_t)ntot;
-    void** bufs[5] = {&b->U, &b->Y0, &b->Y1, &b->acc, &b->V};
-    for (int i = 0; i < 5; ++i)
-        if (dev_malloc(bufs[i], i == 4 ? eb / 2 : eb) != hipSuccess) {
+    struct { void** p; size_t bytes; } bufs[5] = {
+        {&b->U, eb}, {&b->Y0, eb}, {&b->Y1, eb}, {&b->acc, eb + STAGE_PAD}, {&b->V, eb / 2}};
+    for (const auto& q : bufs)
+        if (dev_malloc(q.p, q.bytes) != hipSuccess) {
             nlse_batch_destroy(b);
             return fail(NLSE_ENOMEM, "hipMalloc failed");
         }

@@ -921,8 +921,8 @@ int nlse_create(nlse_solver** out, int dim, int N, int M, int L, int method, int
     h->n = (long)N * M * L;
     const size_t eb = elem_bytes(precision) * (size_t)h->n;
     void** bufs[4] = {&h->U, &h->Y0, &h->Y1, &h->acc};
-    for (void** b : bufs)  // ktot: one point more, for the second half of a staged state of odd size
-        if (dev_malloc(b, eb + (b == &h->acc ? 16 : 0)) != hipSuccess) {
+    for (void** b : bufs)
+        if (dev_malloc(b, eb + (b == &h->acc ? STAGE_PAD : 0)) != hipSuccess) {
             nlse_destroy(h);
             return fail(NLSE_ENOMEM, "hipMalloc failed");
         }

@@ -88,8 +88,11 @@ template <typename T> inline void coefs3d(Coefs<T>& c, T s, T a, T h2, T k)
 
 // Where a resident state lives, for moving it to and from host arrays.  The
 // staging areas are device buffers that hold nothing between steps: s0, s1 and
-// s2 of 8 n, 8 n + 16 and 8 n bytes for single-precision states; s0 of 16 n
-// bytes for double ones.
+// s2 of 8 n, 8 n + STAGE_PAD and 8 n bytes for single-precision states; s0 of
+// 16 n bytes for double ones.  STAGE_PAD: the second half of a state of an odd
+// number of points holds one point more than the first; whoever allocates the
+// buffer handed out as s1 (ktot of solvers and of batches) adds it.
+constexpr size_t STAGE_PAD = 16;
 struct StateRef {
     void *u, *lo, *V;  // lo: low part of a compensated state, else null
     int prec;          // 2 double, 1 single, 3 single with a compensated state

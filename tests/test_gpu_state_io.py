@@ -74,3 +74,29 @@ def test_batch_state_round_trip(hip, prec):
     for p, U in enumerate(Us):
         assert bits_equal(B.state(p), _stored(U, prec))
     B.close()
+
+
+@pytest.mark.parametrize("prec", [2, 3])
+@pytest.mark.parametrize("shape", [(3, 3), (363, 363), (513, 513), (600, 437)])
+def test_one_problem_batch_round_trip(hip, shape, prec):
+    """A batch whose only problem has an odd count (363^2: put above 3 MB, get
+    below; 513^2: both above): the longer half of the staged state has the
+    batch's buffers to itself, with no other problem's points behind it."""
+    print("CASE", shape, prec, flush=True)
+    rng = np.random.default_rng(shape[0] + prec)
+    U = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    V = rng.standard_normal(shape)
+    exp = _stored(U, prec)
+    B = hip.Batch([shape], -1.0, 1.0, 0.01, 0.001, method=1, precision=prec)
+    B.set_state(0, U, V)
+    assert bits_equal(B.state(0), exp)
+    dp = C.POINTER(C.c_double)
+    r, i = np.empty(shape), np.empty(shape)
+    L = hip.lib()
+    assert L.nlse_batch_get_state(B._h, 0, r.ctypes.data_as(dp), i.ctypes.data_as(dp)) == 0
+    assert bits_equal(r + 1j * i, exp)
+    B.set_state(0, np.zeros(shape), V)
+    r[:], i[:] = U.real, U.imag
+    assert L.nlse_batch_set_state(B._h, 0, r.ctypes.data_as(dp), i.ctypes.data_as(dp), V.ctypes.data_as(dp)) == 0
+    assert bits_equal(B.state(0), exp)
+    B.close()
