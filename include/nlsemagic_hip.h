@@ -325,13 +325,16 @@ int nlse_batch_sync(nlse_batch *b);
 /* per-problem diagnostics, out[3p..3p+2] as for nlse_diagnostics */
 int nlse_batch_diagnostics(nlse_batch *b, double *out);
 /* stage kernel family: 0 LDS tiles (rows 8, 16, 32), 1 row-sweep tiles
- * (rows 8, 12, 16; default 16, a whole step per launch), 2 register strips (3..256-row segments, one
- * wave each); see nlse_set_kernel */
+ * (rows 8, 12, 16; default 16), 2 register strips (3..256-row segments, one
+ * wave each); see nlse_set_kernel.  Until nlse_batch_configure sets them, the
+ * stages per launch and the workgroups follow the kernel: a whole step and one
+ * workgroup per tile for row-sweep tiles (double 2SHOC on 8 rows: pairs of
+ * stages), pairs of stages and four workgroups per CU for the others */
 int nlse_batch_set_kernel(nlse_batch *b, int kind, int rows);
 /* stages per launch, kernel kind, rows per tile, workgroups at most */
 int nlse_batch_get_config(const nlse_batch *b, int *fusion, int *kind, int *rows, int *grid);
 /* stages per launch (1, 2, 4), rows per tile (strip segment) of the current kernel family,
- * workgroups at most (a multiple of 8; default: one per tile) and hipGraph steps per replay
+ * workgroups at most (a multiple of 8) and hipGraph steps per replay
  * (0 = off) */
 int nlse_batch_configure(nlse_batch *b, int stages_per_launch, int tile_rows, int grid,
                          int steps_per_graph);

@@ -29,6 +29,7 @@ struct nlse_batch {
     int* tile_prob;  // device: problem of each tile
     int ntiles;
     int fuse, kern, tile, grid;
+    bool configured;  // fuse and grid set by the caller (else default_launch)
     hipStream_t stream;
     hipGraphExec_t gexec[2];
     int gsteps, gcaptured[2];
@@ -75,6 +76,29 @@ int check_rows(int kind, int rows)
                     "batch kernel kind must be 0 (LDS tiles), 1 (row-sweep tiles) or 2 (register strips)");
     }
     return NLSE_OK;
+}
+
+// Stages and workgroups per launch of the current kernel and rows, until the
+// caller sets them.  Row-sweep tiles take a whole RK4 step per launch and a
+// workgroup for every tile, so that the hardware evens out the unequal tiles;
+// LDS tiles and strips pairs of stages on four workgroups per CU that walk the
+// list.  Per step, 2SHOC FP64 MSD, pairs and four workgroups per CU -> whole
+// steps and one per tile: 96 problems of sides 64-512, strips 345 -> 713 us, LDS
+// tiles of 8 rows 353 -> 603; row-sweep tiles of 16 rows 268 -> 200 (FP32c 193 ->
+// 127, CD FP64 203 -> 94, FP32c 138 -> 53).  Row-sweep tiles of 8 rows lose
+// 10-24 % in 2SHOC FP64 on problems of 16-40 points a side (2000 of 32^2 164 ->
+// 202) and keep pairs there.  (Of the gain, by one tile per workgroup instead of
+// a loop over tiles, which keeps registers: 239 -> 217 us 2SHOC FP64, 167 -> 139
+// FP32c.)
+void default_launch(nlse_batch* b)
+{
+    if (b->kern == KERNEL_ROWS) {
+        b->fuse = b->tile == 8 && b->method == 2 && dbl(b) ? 2 : 4;
+        b->grid = GRID_ALL;
+    } else {
+        b->fuse = 2;
+        b->grid = 8 * ((device_cus() * 4 + 7) / 8);
+    }
 }
 
 // (re)build the tile list and per-problem descriptors for the current kernel
@@ -258,18 +282,9 @@ int nlse_batch_create(nlse_batch** out, int nprob, const int* N, const int* M, c
         o += (long)N[p] * M[p];
     }
     b->ntot = ntot;
-    // a whole RK4 step per launch on row-sweep tiles of 16 rows, and a
-    // workgroup for every tile, so that the hardware evens out the unequal
-    // tiles.  Per step, pairs of stages on 8-row tiles with 4 workgroups per CU
-    // -> this: 96 problems of sides 64-512 2SHOC FP64 268 -> 200 us, FP32c 193
-    // -> 127, CD FP64 203 -> 94, FP32c 138 -> 53; 8 problems 2SHOC FP64 36 ->
-    // 27, FP32c 29 -> 19.  (Of that, by one tile per workgroup instead of a
-    // loop over tiles, which keeps registers: 239 -> 217 us 2SHOC FP64, 167 ->
-    // 139 FP32c.)
-    b->fuse = 4;
     b->kern = KERNEL_ROWS;
     b->tile = 16;
-    b->grid = GRID_ALL;
+    default_launch(b);
     const size_t eb = (precision == 2 ? 16 : 8) * (size_t)ntot;
     struct { void** p; size_t bytes; } bufs[5] = {
         {&b->U, eb}, {&b->Y0, eb}, {&b->Y1, eb}, {&b->acc, eb + STAGE_PAD}, {&b->V, eb / 2}};
@@ -422,6 +437,7 @@ int nlse_batch_set_kernel(nlse_batch* b, int kind, int rows)
     if (rc != NLSE_OK) return rc;
     b->kern = kind;
     b->tile = rows;
+    if (!b->configured) default_launch(b);
     return build_tiles(b);
 }
 
@@ -444,6 +460,7 @@ int nlse_batch_configure(nlse_batch* b, int stages_per_launch, int tile_rows, in
     if (rc != NLSE_OK) return rc;
     if (grid < 8 || grid % 8 != 0) return fail(NLSE_EINVAL, "grid must be a positive multiple of 8");
     if (steps_per_graph < 0) return fail(NLSE_EINVAL, "steps per graph must be >= 0");
+    b->configured = true;
     b->grid = grid;
     b->gsteps = steps_per_graph;
     drop_graphs(b);
@@ -474,6 +491,7 @@ int nlse_batch_autotune(nlse_batch* b, int steps, int* best_fusion, int* best_ti
     const int tl[3][3] = {{8, 16, 32}, {8, 12, 16}, {16, 32, 64}};
     const int gsave = b->gsteps;
     const int of = b->fuse, ok = b->kern, ot = b->tile, og = b->grid;  // restored if a trial fails
+    const bool oc = b->configured;
     int bf = of, bk = ok, bt = ot, bg = og, rc = NLSE_OK;
     double bms = 1e30;
     for (int kind = 0; kind < 3 && rc == NLSE_OK; ++kind)
@@ -502,6 +520,7 @@ int nlse_batch_autotune(nlse_batch* b, int steps, int* best_fusion, int* best_ti
     if (saved_lo) (void)hipFree(saved_lo);
     if (rc != NLSE_OK) {  // the batch keeps the configuration it had; the trial's error is reported
         if (nlse_batch_set_kernel(b, ok, ot) == NLSE_OK) (void)nlse_batch_configure(b, of, ot, og, gsave);
+        b->configured = oc;
         return rc;
     }
     rc = nlse_batch_set_kernel(b, bk, bt);

@@ -43,3 +43,33 @@ def test_batch_tiles(oracle, method, precision, BC, grid):
         if precision == 2:
             assert bits_equal(B.state(i), oracle.take_steps(U[i], V[i], s[i], a[i], h2[i], BC, 3, k[i], method)), SHAPES[i]
     B.close()
+
+
+@pytest.mark.parametrize("kind,rows,fusion", [(0, 8, 2), (0, 16, 2), (0, 32, 2), (2, 16, 2), (1, 8, 2), (1, 12, 4),
+                                              (1, 16, 4)])
+def test_launch_follows_kernel_until_configured(kind, rows, fusion):
+    """Choosing a kernel family takes that family's stages and workgroups per
+    launch; what configure() set stays."""
+    import nlsemagic_amd as nm
+    print("CASE batch launch", kind, rows, flush=True)
+    B = nm.Batch([(40, 50), (33, 97)], -1.0, 1.0, 0.04, 0.003, method=2, precision=2)
+    assert B.config()[:3] == (4, 1, 16)
+    every = B.config()[3]  # a workgroup for every tile
+    B.set_kernel(kind, rows)
+    assert B.config()[:3] == (fusion, kind, rows)
+    assert (B.config()[3] == every) == (kind == 1)
+    B.set_kernel(1, 16)
+    assert B.config() == (4, 1, 16, every)
+    B.configure(1, 16, 64, 0)
+    B.set_kernel(kind, rows)
+    assert B.config() == (1, kind, rows, 64)
+    B.close()
+
+
+def test_single_precision_keeps_whole_steps_on_8_rows():
+    import nlsemagic_amd as nm
+    for method, precision in ((1, 2), (1, 3), (2, 3)):
+        B = nm.Batch([(40, 50)], -1.0, 1.0, 0.04, 0.003, method=method, precision=precision)
+        B.set_kernel(1, 8)
+        assert B.config()[0] == 4, (method, precision)
+        B.close()
