@@ -100,3 +100,33 @@ def test_one_problem_batch_round_trip(hip, shape, prec):
     assert L.nlse_batch_set_state(B._h, 0, r.ctypes.data_as(dp), i.ctypes.data_as(dp), V.ctypes.data_as(dp)) == 0
     assert bits_equal(B.state(0), exp)
     B.close()
+
+
+# points whose put (24 B each) or get (16 B) lies below or at 256 KB, from where
+# a single-precision state passes the pinned block as floats, and whose floats
+# (12 B, 8 B) fill a block or just do not
+@pytest.mark.parametrize("n", [10922, 10923, 16383, 16384, 262144, 262145, 393216, 393217])
+def test_single_precision_through_the_block(hip, n):
+    print("CASE", n, flush=True)
+    rng = np.random.default_rng(n)
+    U = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    U[:6] = [np.inf, -np.inf, 1e-50, 1e50, 3e-42 + 1e39j, -0.0]  # kept, underflowing, overflowing, subnormal
+    U[-1] = complex(1 + 2.0 ** -24, np.nan)                      # a tie
+    V = rng.standard_normal(n)
+    with np.errstate(over="ignore", invalid="ignore"):
+        exp = U.astype(np.complex64).astype(np.complex128)
+    sol = hip.Solver((n,), 1, 1, 1, -1.0, 1.0, 0.01, 0.001)
+    dp = C.POINTER(C.c_double)
+    L = hip.lib()
+    r, i, v = np.ascontiguousarray(U.real), np.ascontiguousarray(U.imag), V
+    gr, gi = np.empty(n), np.empty(n)
+    for put in (lambda: sol.set_state(U, V), lambda: sol.set_state(U),
+                lambda: L.nlse_set_state(sol._h, *(x.ctypes.data_as(dp) for x in (r, i, v)))):
+        sol.set_state(np.zeros(n))
+        put()
+        assert bits_equal(sol.state(), exp)
+        assert L.nlse_get_state(sol._h, gr.ctypes.data_as(dp), gi.ctypes.data_as(dp)) == 0
+        assert bits_equal(gr, exp.real.copy()) and bits_equal(gi, exp.imag.copy())
+    sol.fill(1.0)
+    assert abs(sol.energy()[2] / 0.1 - (V.astype(np.float32).astype(float).sum() + 0.5 * n)) < 1e-9 * n
+    sol.close()
