@@ -302,6 +302,17 @@ for _dim in (1, 2, 3):
             __all__.append(_n)
 
 
+def _put(complex_entry, planes_entry, head, U, v):
+    """A state to the device: complex arrays interleaved, real ones as their
+    one plane (no complex copy of them is made)."""
+    if np.iscomplexobj(U):
+        u = np.ascontiguousarray(U, dtype=np.complex128)
+        _check(complex_entry(*head, u.ctypes.data, v.ctypes.data if v is not None else None))
+    else:
+        u = np.ascontiguousarray(U, dtype=np.float64)
+        _check(planes_entry(*head, _p(u, C.c_double), None, _p(v, C.c_double) if v is not None else None))
+
+
 class Solver:
     """Device-resident RK4 integrator (the nlse_create/... C ABI).
 
@@ -336,13 +347,12 @@ class Solver:
         U = np.asarray(U)
         if U.shape != self.shape:
             raise ValueError("shape mismatch")
-        u = np.ascontiguousarray(U, dtype=np.complex128)
         v = None
         if V is not None:
             v = np.ascontiguousarray(V, dtype=np.float64)
             if v.shape != self.shape:
                 raise ValueError("shape mismatch")
-        _check(self._lib.nlse_set_state_z(self._h, u.ctypes.data, v.ctypes.data if v is not None else None))
+        _put(self._lib.nlse_set_state_z, self._lib.nlse_set_state, (self._h,), U, v)
 
     def state(self):
         out = np.empty(self.shape, np.complex128)
@@ -583,9 +593,8 @@ class Batch:
         U = np.asarray(U)
         if U.shape != self.shapes[p]:
             raise ValueError("shape mismatch")
-        u = np.ascontiguousarray(U, dtype=np.complex128)
         v = np.ascontiguousarray(V, dtype=np.float64) if V is not None else None
-        _check(self._lib.nlse_batch_set_state_z(self._h, int(p), u.ctypes.data, v.ctypes.data if v is not None else None))
+        _put(self._lib.nlse_batch_set_state_z, self._lib.nlse_batch_set_state, (self._h, int(p)), U, v)
 
     def state(self, p):
         out = np.empty(self.shapes[p], np.complex128)

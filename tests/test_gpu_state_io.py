@@ -130,3 +130,40 @@ def test_single_precision_through_the_block(hip, n):
     sol.fill(1.0)
     assert abs(sol.energy()[2] / 0.1 - (V.astype(np.float32).astype(float).sum() + 0.5 * n)) < 1e-9 * n
     sol.close()
+
+
+@pytest.mark.parametrize("prec", [2, 1, 3])
+@pytest.mark.parametrize("n", [401, 400001])
+def test_real_states_go_without_a_complex_copy(hip, n, prec):
+    """A real array is a state with no imaginary part, whatever the state held
+    before, and is handed over as it is."""
+    import tracemalloc
+    print("CASE", n, prec, flush=True)
+    rng = np.random.default_rng(n + prec)
+    U = rng.standard_normal(n)
+    sol = hip.Solver((n,), 1, prec, 1, -1.0, 1.0, 0.01, 0.001)
+    for real in (U, U.astype(np.float32), np.arange(n) % 7, np.arange(n) % 2 == 0, U[::-1]):
+        sol.set_state(rng.standard_normal(n) + 1j)
+        tracemalloc.start()
+        sol.set_state(real)
+        peak = tracemalloc.get_traced_memory()[1]
+        tracemalloc.stop()
+        assert bits_equal(sol.state(), _stored(real.astype(np.float64) + 0j, prec))
+        as_is = real.dtype == np.float64 and real.flags.c_contiguous
+        assert peak < 20000 + (0 if as_is else 8 * n)
+    sol.close()
+
+
+@pytest.mark.parametrize("prec", [2, 3])
+def test_real_batch_states(hip, prec):
+    shapes = [(301, 437), (37, 64)]
+    rng = np.random.default_rng(prec)
+    B = hip.Batch(shapes, -1.0, 1.0, 0.01, 0.001, method=1, precision=prec)
+    for p, sh in enumerate(shapes):
+        B.set_state(p, rng.standard_normal(sh) + 1j, np.zeros(sh))
+    Us = [rng.standard_normal(sh) for sh in shapes]
+    for p, U in enumerate(Us):
+        B.set_state(p, U, np.zeros(U.shape))
+    for p, U in enumerate(Us):
+        assert bits_equal(B.state(p), _stored(U + 0j, prec))
+    B.close()
