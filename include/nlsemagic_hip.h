@@ -378,6 +378,11 @@ int nlse_device_count(void);
  * chunk loop with per-chunk diagnostics allocates nothing after its first
  * call */
 long long nlse_device_allocations(void);
+/* number of pinned host allocations the library has made since it was loaded:
+ * the solvers' result slots (one allocation, with the first solver), blocks of
+ * 3 MB for states (16 at most), and the chunks of larger copies (3 of 4 MB per
+ * device); all are kept */
+long long nlse_pinned_allocations(void);
 
 #ifdef __cplusplus
 }

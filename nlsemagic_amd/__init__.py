@@ -145,6 +145,8 @@ def lib():
     L.nlse_energy.argtypes = [C.c_void_p, _D]
     L.nlse_device_allocations.restype = C.c_longlong
     L.nlse_device_allocations.argtypes = []
+    L.nlse_pinned_allocations.restype = C.c_longlong
+    L.nlse_pinned_allocations.argtypes = []
     L.nlse_group_create.restype = C.c_int
     L.nlse_group_create.argtypes = [C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.c_int]
     L.nlse_group_step.restype = C.c_int
@@ -777,3 +779,9 @@ def device_allocations():
     """Device allocations the library has made since it was loaded (see
     nlse_device_allocations)."""
     return int(lib().nlse_device_allocations())
+
+
+def pinned_allocations():
+    """Pinned host allocations the library has made since it was loaded (see
+    nlse_pinned_allocations)."""
+    return int(lib().nlse_pinned_allocations())

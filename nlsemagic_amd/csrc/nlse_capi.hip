@@ -29,7 +29,7 @@ int set_error(int code, const std::string& msg)
     return code;
 }
 
-std::atomic<long long> g_allocs{0};
+std::atomic<long long> g_allocs{0}, g_pinned{0};
 
 // compute units of the current device
 int device_cus()
@@ -53,6 +53,47 @@ hipError_t dev_malloc_raw(void** p, size_t bytes)
 }
 
 namespace {
+
+// every pinned allocation (nlse_pinned_allocations reports the count)
+hipError_t pin_malloc(char** p, size_t bytes)
+{
+    ++g_pinned;
+    return hipHostMalloc((void**)p, bytes, hipHostMallocPortable | hipHostMallocMapped);
+}
+
+// Pinned result slots, one per solver, which its reductions write directly:
+// taken when a solver is created and given back when it is destroyed, all from
+// one allocation made with the first solver.  Solvers beyond SLOTS have none
+// (null) and copy their results.
+constexpr int SLOTS = 128, SLOT_DOUBLES = 8;
+std::mutex g_slot_mu;
+double* g_slots = nullptr;
+bool g_slots_tried = false;
+int g_slot_free[SLOTS];
+int g_slots_free = 0;
+
+double* take_slot()
+{
+    std::lock_guard<std::mutex> lk(g_slot_mu);
+    if (!g_slots_tried) {
+        g_slots_tried = true;
+        char* q = nullptr;
+        if (pin_malloc(&q, sizeof(double) * SLOT_DOUBLES * SLOTS) == hipSuccess) {
+            g_slots = (double*)q;
+            for (int i = 0; i < SLOTS; ++i) g_slot_free[i] = SLOTS - 1 - i;
+            g_slots_free = SLOTS;
+        } else {
+            (void)hipGetLastError();
+        }
+    }
+    return g_slots_free ? g_slots + SLOT_DOUBLES * g_slot_free[--g_slots_free] : nullptr;
+}
+void give_slot(double* p)
+{
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(g_slot_mu);
+    g_slot_free[g_slots_free++] = (int)((p - g_slots) / SLOT_DOUBLES);
+}
 
 // host threads that split one memcpy between them
 class CopyPool {
@@ -168,7 +209,7 @@ bool staging_ready(Staging& S, int dev)
               hipEventCreateWithFlags(&S.after, hipEventDisableTiming) == hipSuccess &&
               hipEventCreateWithFlags(&S.done, hipEventDisableTiming) == hipSuccess;
     for (int i = 0; i < XFER_SLOTS && ok; ++i) {
-        ok = hipHostMalloc((void**)&S.pin[i], XFER_CHUNK, hipHostMallocDefault) == hipSuccess &&
+        ok = pin_malloc(&S.pin[i], XFER_CHUNK) == hipSuccess &&
              hipEventCreateWithFlags(&S.ev[i], hipEventDisableTiming) == hipSuccess;
     }
     if (hipSetDevice(cur) != hipSuccess || !ok) return false;
@@ -381,10 +422,10 @@ PinnedBlock::PinnedBlock() : p_(nullptr)
         p_ = g_pin_free.back();
         g_pin_free.pop_back();
     } else if (g_pin_made < PIN_BLOCKS) {
-        void* q = nullptr;
-        if (hipHostMalloc(&q, SIZE, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+        char* q = nullptr;
+        if (pin_malloc(&q, SIZE) == hipSuccess) {
             ++g_pin_made;
-            p_ = (char*)q;
+            p_ = q;
         } else {
             (void)hipGetLastError();
         }
@@ -564,6 +605,7 @@ struct nlse_solver {
     // profile), allocated with the solver: those calls allocate nothing
     double* ws;
     long ws_len;  // doubles
+    double* res;  // pinned slot for a reduction's results (null: none free)
 };
 
 namespace {
@@ -811,12 +853,11 @@ StateRef state_ref(const nlse_solver* h)
     return StateRef{h->U, h->Ulo, h->V, h->prec, h->n, h->Y0, h->acc, h->Y1, h->stream};
 }
 
-// values of a reduction that leaves m doubles at its `out`: reduced straight
-// into pinned memory where there is some, else into `dev` and copied
+// values of a reduction that leaves m <= SLOT_DOUBLES doubles at its `out`:
+// reduced straight into the solver's pinned slot, else into `dev` and copied
 template <typename F> int fetch(nlse_solver* h, const char* what, int m, double* dev, double* out, F&& launch)
 {
-    PinnedBlock blk;
-    double* const d = blk.get() ? (double*)blk.get() : dev;
+    double* const d = h->res ? h->res : dev;
     hipError_t e = launch(d);
     if (e == hipSuccess && d == dev)
         e = hipMemcpyAsync(out, dev, sizeof(double) * m, hipMemcpyDeviceToHost, h->stream);
@@ -917,6 +958,8 @@ const char* nlse_last_error(void) { return g_err.c_str(); }
 
 long long nlse_device_allocations(void) { return g_allocs.load(); }
 
+long long nlse_pinned_allocations(void) { return g_pinned.load(); }
+
 int nlse_device_count(void)
 {
     int n = 0;
@@ -977,6 +1020,7 @@ int nlse_create(nlse_solver** out, int dim, int N, int M, int L, int method, int
         nlse_destroy(h);
         return fail(NLSE_EHIP, "stream/event creation failed");
     }
+    h->res = take_slot();
     h->ubase = h->U;
     // 2D: a whole RK4 step per launch on row-sweep tiles of 16 rows (on a
     // 1024^2 MSD grid 8-55 % faster than pairs of stages on 8-row tiles,
@@ -1010,6 +1054,7 @@ void nlse_destroy(nlse_solver* h)
     void* bufs[8] = {h->U, h->Y0, h->Y1, h->acc, h->D, h->V, h->Ulo, h->ws};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
+    give_slot(h->res);
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
