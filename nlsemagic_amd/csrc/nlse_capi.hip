@@ -408,19 +408,18 @@ template <typename S> bool rounded(const StateRef& h, size_t bytes)
     return sizeof(S) == 8 && h.prec == 1 && bytes >= ROUND_MIN;
 }
 
-std::mutex g_pin_mu;
-std::vector<char*> g_pin_free;
-int g_pin_made = 0;
 constexpr int PIN_BLOCKS = 16;
+std::mutex g_pin_mu;
+char* g_pin_free[PIN_BLOCKS];  // an array: giving a block back neither allocates nor throws
+int g_pin_nfree = 0, g_pin_made = 0;
 
 }  // namespace
 
 PinnedBlock::PinnedBlock() : p_(nullptr)
 {
     std::lock_guard<std::mutex> lk(g_pin_mu);
-    if (!g_pin_free.empty()) {
-        p_ = g_pin_free.back();
-        g_pin_free.pop_back();
+    if (g_pin_nfree > 0) {
+        p_ = g_pin_free[--g_pin_nfree];
     } else if (g_pin_made < PIN_BLOCKS) {
         char* q = nullptr;
         if (pin_malloc(&q, SIZE) == hipSuccess) {
@@ -435,7 +434,7 @@ PinnedBlock::~PinnedBlock()
 {
     if (!p_) return;
     std::lock_guard<std::mutex> lk(g_pin_mu);
-    g_pin_free.push_back(p_);
+    g_pin_free[g_pin_nfree++] = p_;
 }
 
 namespace {
