@@ -126,16 +126,24 @@ __global__ __launch_bounds__(256) void batch_diag_fold_kernel(const double* __re
 int diag_blocks(long n) { return (int)std::min<long>(DIAG_BLOCKS, (n + 255) / 256); }
 
 // the diagnostics of every problem of a batch (table `probs`, state in buffer
-// r_u) into out[3p ..]: two launches for all of them instead of two each, with
-// the partials each problem has alone, so the bits are the same; part0: prefix
-// sums of diag_blocks, nprob + 1 values
+// r_u) into out[3p ..]: two launches for up to 65535 of them (problems are the
+// grid's y axis, which holds no more) instead of two each, with the partials
+// each problem has alone, so the bits are the same; part0: prefix sums of
+// diag_blocks, nprob + 1 values
 template <typename T>
 hipError_t launch_batch_diag(const BatchProb2<T>* probs, int nprob, int r_u, int maxblocks, const int* part0,
                              double* part, double* out, hipStream_t st)
 {
-    hipLaunchKernelGGL((batch_diag_partial_kernel<T>), dim3(maxblocks, nprob), dim3(256), 0, st, probs, r_u, part0, part);
-    hipLaunchKernelGGL(batch_diag_fold_kernel, dim3(nprob), dim3(256), 0, st, part, part0, out);
-    return hipGetLastError();
+    constexpr int SLICE = 65535;
+    for (int p = 0; p < nprob; p += SLICE) {
+        const int n = std::min(SLICE, nprob - p);
+        hipLaunchKernelGGL((batch_diag_partial_kernel<T>), dim3(maxblocks, n), dim3(256), 0, st, probs + p, r_u,
+                           part0 + p, part);
+        hipLaunchKernelGGL(batch_diag_fold_kernel, dim3(n), dim3(256), 0, st, part, part0 + p, out + 3 * (long)p);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 template hipError_t launch_batch_diag<double>(const BatchProb2<double>*, int, int, int, const int*, double*, double*,
                                               hipStream_t);

@@ -73,3 +73,23 @@ def test_single_precision_keeps_whole_steps_on_8_rows():
         B.set_kernel(1, 8)
         assert B.config()[0] == 4, (method, precision)
         B.close()
+
+
+@pytest.mark.parametrize("precision", [2, 3])
+def test_diagnostics_of_more_problems_than_a_grid_axis(precision):
+    """70,000 problems of 3 x 3 and one larger one: more than the 65,535 that
+    one launch of the batch reductions takes."""
+    import nlsemagic_amd as nm
+    print("CASE batch diagnostics", precision, flush=True)
+    n, big = 70_000, 65_540
+    shapes = [(3, 3)] * n
+    shapes[big] = (40, 33)
+    B = nm.Batch(shapes, -1.0, 1.0, 0.04, 0.003, method=1, precision=precision)
+    exp = np.zeros((n, 3))
+    rng = np.random.default_rng(precision)
+    for p in (0, 1, 65_533, 65_534, 65_535, 65_536, big, n - 1):
+        U = rng.integers(-8, 9, shapes[p]) + 1j * rng.integers(-8, 9, shapes[p])  # sums of squares: exact
+        B.set_state(p, U, np.zeros(shapes[p]))
+        exp[p] = (U.real ** 2 + U.imag ** 2).sum(), U.real.max(), 0
+    assert np.array_equal(B.diagnostics(), exp)
+    B.close()
