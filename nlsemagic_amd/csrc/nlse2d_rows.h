@@ -102,8 +102,10 @@ struct RowsLds {
 // The F phase then reads no Y but the row's own, so each row's new Y goes to LDS
 // at once and a stage has two barriers instead of three.  FP64 whole steps on 8
 // waves, per step: 1024^2 30.9 -> 28.8 us (MSD 31.9 -> 30.0), 700^2 18.7 -> 17.2,
-// 512^2 10.8 -> 10.5, 96 problems of sides 64-512 204 -> 194.  On 16 waves, where
-// a launch is one round of tiles, MSD loses (131 x 150 10.5 -> 10.8), and single
+// 512^2 10.8 -> 10.5, 96 problems of sides 64-512 204 -> 194.  Not in tiles with
+// the grid's first or last rows, which set the time of a launch of one round:
+// MSD 560^2 16.9 us with it, 15.9 without, 600^2 16.0 and 14.8, 64^2 on 16 rows
+// 15.7 and 15.0.  On 16 waves MSD loses (131 x 150 10.5 -> 10.8), and single
 // precision gains nothing at 1024^2 and loses up to 3 % below.  The row's own D
 // held as well: 47-56 registers spilled, 96 problems 210 us.
 template <typename T, int METHOD, int FIRST, int LAST, int NW> constexpr bool rows_early()
@@ -172,7 +174,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
         return colL ? p : (colR ? m : v);
     };
 
-    constexpr bool EARLY = rows_early<T, METHOD, FIRST, LAST, NW>();
+    constexpr bool EARLY = RIN && rows_early<T, METHOD, FIRST, LAST, NW>();
 
     // rows of this wave: e = 4k + w; everything about row e stays in slot k
     c2<T> Yc[RW], Uc[RW], Ac[RW], Lc[RW];
@@ -240,13 +242,9 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 const int g = g0 + e;
                 const c2<T> yx = Yc[k];
                 if (EARLY && e >= flo && e < fhi) {
-                    if (interior(g)) {
-                        const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
-                        Gc[k] = mk<T>(aa.x + ab.x - 4 * yx.x + ba.x + bb.x, aa.y + ab.y - 4 * yx.y + ba.y + bb.y);
-                        pin_here<T>(Gc[k]);
-                    } else if (msd) {
-                        ypart[k] = sy(g == 0 ? e + 1 : e - 1, 0);
-                    }
+                    const c2<T> aa = sy(e + 1, 1), ab = sy(e + 1, -1), ba = sy(e - 1, 1), bb = sy(e - 1, -1);
+                    Gc[k] = mk<T>(aa.x + ab.x - 4 * yx.x + ba.x + bb.x, aa.y + ab.y - 4 * yx.y + ba.y + bb.y);
+                    pin_here<T>(Gc[k]);
                 }
                 const T vx = Vc[k];
                 c2<T> dd = z;
@@ -380,7 +378,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
             } else if (BC == BC_LAP0) {
                 ff = lap0_f<T>(yx, vx, c.s);
             } else if (msd) {  // row 0 or N-1: F after the barrier
-                if (!EARLY) ypart[k] = sy(g == 0 ? e + 1 : e - 1, 0);
+                ypart[k] = sy(g == 0 ? e + 1 : e - 1, 0);
                 continue;
             }
             epilogue(k, e, ff);
@@ -389,7 +387,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
         }
         // every read of this stage's Y and D rows is done (after the last
         // stage only the MSD boundary rows below still read LDS; EARLY: the new Y
-        // rows are in LDS, but for rows 0 and N-1)
+        // rows are in LDS)
         if (q < NF - 1 || top || bot) __syncthreads();
         if (top || bot) {
 #pragma unroll
@@ -399,7 +397,6 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 const int g = g0 + e;
                 if (g == 0) epilogue(k, e, msd_f<T>(colq(sm.y[1 + lane]), colq(ypart[k]), Yc[k]));
                 else if (g == N - 1) epilogue(k, e, msd_f<T>(colq(sm.y[1 + (TE - 1) * 64 + lane]), colq(ypart[k]), Yc[k]));
-                if (EARLY && q < NF - 1 && (g == 0 || g == N - 1)) sm.y[1 + e * 64 + lane] = Yc[k];
             }
         }
         if (!EARLY && q < NF - 1) {
@@ -409,7 +406,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
                 if (e >= flo && e < fhi) sm.y[1 + e * 64 + lane] = Yc[k];
             }
         }
-        if (q < NF - 1 && (!EARLY || top || bot)) __syncthreads();  // the next stage's input rows are in LDS
+        if (!EARLY && q < NF - 1) __syncthreads();  // the next stage's input rows are in LDS
     }
 }
 
