@@ -139,17 +139,22 @@ static hipError_t launch_rows_ti(const StageArgs<T>& a, hipStream_t st)
 // Whole-step tiles by grid size.  A launch with few tiles takes one tile's
 // time, which shorter tiles and more waves cut; once the tiles come in several
 // rounds the work of their halo rows counts instead.  The lines, in tiles per
-// CU of 8, 12 and 16 rows, from a sweep of 12 grids (100^2 to 1024^2, both
-// methods, all precisions, Dirichlet and MSD; per step, 16 rows on 8 waves ->
-// the choice):
+// CU of 8, 12 and 16 rows, from sweeps of 41 grids (64^2 to 2048^2, and 3 to
+// 20000 points a side; both methods, all precisions, Dirichlet and MSD; per
+// step, 16 rows on 8 waves -> the choice):
 //   8 rows on 16 waves   100^2 CD FP64 6.7 -> 4.7 us, 2SHOC FP64 11.3 -> 8.0
-//                        (MSD 14.4 -> 10.3), 448^2 CD FP32 MSD 7.7 -> 5.2
-//   8 rows on 8 waves    384^2 2SHOC FP64 11.7 -> 9.9, 512^2 2SHOC FP32 10.0 ->
-//                        8.4, 600^2 CD FP32c MSD 8.2 -> 6.6
-//   12 rows on 8 waves   512^2 2SHOC FP64 12.2 -> 10.8
-//   16 rows on 16 waves  600^2 2SHOC FP32 10.2 -> 8.6; 1000 x 100 2SHOC FP64
-//                        10.2 (two of three tiles hold a boundary: 8 rows 12.6)
-//   16 rows on 8 waves   from 700^2 on (8 rows there: 2SHOC FP64 18.0 -> 21.4)
+//                        (MSD 14.4 -> 10.3), 448^2 CD FP32 MSD 7.7 -> 5.2; CD on
+//                        at most 32 rows only while there is a tile per CU
+//                        (3 x 20000 CD FP32 4.6 -> 5.1, on 8 waves 4.3)
+//   8 rows on 8 waves    384^2 2SHOC FP64 11.4 -> 8.9, 512^2 2SHOC FP32 9.3 ->
+//                        7.9, 600^2 CD FP32c MSD 8.2 -> 6.6; CD FP64 up to 3.8
+//                        tiles per CU (2000 x 200, 3.9: 7.2 -> 8.5)
+//   12 rows on 8 waves   512^2 2SHOC FP64 11.6 -> 10.2, 600^2 2SHOC FP32 MSD
+//                        12.4 -> 11.3 (16 rows on 16 waves 13.0)
+//   16 rows on 16 waves  2SHOC on few rows or columns, where most tiles hold a
+//                        boundary: 1000 x 100 2SHOC FP64 10.7 -> 9.4 (8 rows
+//                        10.0), 17 x 5000 9.4 -> 8.1 (8 rows 9.9)
+//   16 rows on 8 waves   from 700^2 on (8 rows there: 2SHOC FP64 16.4 -> 19.9)
 struct RowsChoice {
     int rows, waves;
 };
@@ -159,16 +164,15 @@ static RowsChoice rows_choice(int method, bool dbl, int N, int M)
     const long cols = (M + (M % W == 1) + W - 1) / W;
     auto tiles = [&](int TI) { return cols * ((N + (N % TI == 1) + TI - 1) / TI); };
     const long cus = device_cus();
+    if (tiles(8) <= cus) return {8, 16};
     if (method == 1) {
-        if (tiles(8) <= 2 * cus) return {8, 16};
-        if (tiles(8) <= 4 * cus) return {8, 8};
+        if (10 * tiles(8) <= 19 * cus && N > 32) return {8, 16};
+        if (10 * tiles(8) <= (dbl ? 38 : 40) * cus) return {8, 8};
         return {16, 8};
     }
-    if (tiles(8) <= cus) return {8, 16};
-    if (cols <= 3 && tiles(16) <= cus) return {16, 16};
+    if ((cols <= 3 || N <= 32) && tiles(16) <= cus) return {16, 16};
     if (4 * tiles(8) <= (dbl ? 9 : 12) * cus) return {8, 8};
-    if (dbl && tiles(12) <= 2 * cus) return {12, 8};
-    if (!dbl && tiles(16) <= 2 * cus) return {16, 16};
+    if (tiles(dbl ? 12 : 16) <= 2 * cus) return {12, 8};
     return {16, 8};
 }
 
