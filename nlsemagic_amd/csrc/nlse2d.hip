@@ -179,7 +179,9 @@ static RowsChoice rows_choice(int method, bool dbl, int N, int M)
 int default_rows2d(int method, bool dbl, int N, int M) { return rows_choice(method, dbl, N, M).rows; }
 
 // a whole step on tiles of a.tile rows: the waves of the choice where it has
-// these rows, else 16 waves while there is at most one tile per CU
+// these rows, else 16 waves while there is at most one tile per CU.  8 rows of CD
+// that the caller asked for on a larger grid take 4 waves (1024^2 FP32 8.0 us,
+// 8 waves 9.5; 2048^2 23.5 and 31.4)
 template <typename T, int METHOD>
 static hipError_t launch_rows_step(const StageArgs<T>& a, hipStream_t st)
 {
@@ -192,6 +194,8 @@ static hipError_t launch_rows_step(const StageArgs<T>& a, hipStream_t st)
     case 16:
         return NW == 16 ? launch_rows_ti<T, METHOD, 1, 4, 16, 16>(a, st) : launch_rows_ti<T, METHOD, 1, 4, 16, 8>(a, st);
     default:
+        if constexpr (METHOD == 1)
+            if (NW != 16 && c.rows != 8) return launch_rows_ti<T, METHOD, 1, 4, 8, 4>(a, st);
         return NW == 16 ? launch_rows_ti<T, METHOD, 1, 4, 8, 16>(a, st) : launch_rows_ti<T, METHOD, 1, 4, 8, 8>(a, st);
     }
 }
