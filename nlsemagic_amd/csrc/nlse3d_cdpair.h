@@ -165,8 +165,14 @@ __device__ __forceinline__ void cdpair_tile(Lds& sm, int i0, int j0, int k0, con
         }
     };
     // the second stage's update of the point pp from its F, ktot so far, base
-    // U and (compensated) low part
-    auto fin2 = [&](long pp, c2<T> f, c2<T> a, c2<T> b, c2<T> lo) {
+    // U and (compensated) low part.  By reference without MSD: by value, stages 3-4
+    // in FP32 take 66 registers instead of 64, and a CU holds one workgroup instead
+    // of two (900 x 1001 x 3 CD FP32 per step 529 -> 445 us, 512 x 512 x 16 174 ->
+    // 154, 3 x 1001 x 900 72 -> 66, 256^3 279 -> 273).  MSD has one either way, and
+    // by reference FP32 compensated loses 7 % (256^3 357 -> 384).
+    using Arg = std::conditional_t<MSD, c2<T>, const c2<T>&>;
+    auto fin2 = [&](long pp, Arg f, Arg ktot, Arg base, Arg low) {
+        c2<T> a = ktot, b = base;
         if constexpr (!SECOND) {
             // stage 2: ktot = K1 + 2 K2, Y2 = U + k/2 K2
             a.x = a.x + (T)2.0 * f.x;
@@ -178,6 +184,7 @@ __device__ __forceinline__ void cdpair_tile(Lds& sm, int i0, int j0, int k0, con
             a.x = a.x + (T)1.0 * f.x;
             a.y = a.y + (T)1.0 * f.y;
             if (HAS_LO && ulo) {
+                c2<T> lo = low;
                 comp_add<T>(b.x, lo.x, c.k6 * a.x);
                 comp_add<T>(b.y, lo.y, c.k6 * a.y);
                 st_stream<T>(&ulo[pp], lo);
