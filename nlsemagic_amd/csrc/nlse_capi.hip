@@ -644,7 +644,11 @@ void drop_graphs(nlse_solver* h)
 // a second barrier and a division per stencil, and small grids are all
 // boundary.  Per step, one stage / two: CD FP64 64^3 22 / 28 us, 80^3 45 / 29;
 // 2SHOC FP32c 64^3 48 / 55, 80^3 107 / 76; 2SHOC FP64 (4-row tiles) 64^3 54 /
-// 67, 97 x 120 x 111 203 / 173, 128^3 261 / 307, 157 x 149 x 163 642 / 371.
+// 67, 132^3 357 / 285, 157 x 149 x 163 643 / 371.  Below, 2SHOC FP64 goes either way
+// as the tiles fall (97 x 120 x 111 200 / 146, 120^3 240 / 252, 128^3 260 / 307), and
+// one stage stays.  Above the lines pairs lose only on a second axis shorter than
+// a tile's 12 rows, most of whose waves idle (256 x 8 x 256 CD FP32 26 / 32, 1001 x
+// 3 x 900 83 / 134; 256 x 13 x 256 43 / 41).
 bool msd_pairs(const nlse_solver* h)
 {
     return h->n >= (h->method == 2 && h->prec == 2 ? 2500000 : 400000);
