@@ -328,7 +328,7 @@ __device__ __forceinline__ void cdpair_tile(Lds& sm, int i0, int j0, int k0, con
             }
             // (d) MSD rows 0 and N-1 of both stages' planes, from the om their
             // partner rows left in LDS
-            if (jbc) {
+            if constexpr (MSD) if (jbc) {
                 __syncthreads();
 #pragma unroll
                 for (int r = 0; r < RW; ++r) {

@@ -537,7 +537,7 @@ struct ShocPair {
                 constexpr int u4 = decltype(uc)::value;
                 const int p = pstart + q0 + u4;
                 (step<u4>(R, p), ...);
-                if (jbc) {
+                if constexpr (MSD) if (jbc) {
                     __syncthreads();
                     (edge_row<u4>(R, p), ...);
                 }
