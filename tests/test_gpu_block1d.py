@@ -42,3 +42,29 @@ def test_block1d_every_tail_matches_oracle(hip, oracle, n, method):
                 got = hip.take_steps(U, V, -1.0, 0.9, 0.04, BC, steps, 0.004, precision=prec, method=method)
                 exp = oracle.take_steps(U, V, -1.0, 0.9, 0.04, BC, steps, 0.004, method, precision=prec)
                 assert bits_equal(got, exp), (BC, prec, steps)
+
+
+@pytest.mark.parametrize("method", [1, 2])
+@pytest.mark.parametrize("n", SIZES)
+def test_block1d_compensated_matches_unblocked(hip, n, method):
+    """Compensated states: the bits of the kernels without windows (the whole
+    chunk in one workgroup, or a launch per stage above 4096 points), for a
+    chunk of several launches and an odd one after it."""
+    rng = np.random.default_rng(n + method)
+    U = (0.9 + 0.3 * rng.uniform(-1, 1, n)) + 1j * (0.3 * rng.uniform(-1, 1, n))
+    V = 0.5 * rng.uniform(-1, 1, n)
+    for BC in (1, 2, 3, 4, 0):
+        if BC == 4 and n < 4:
+            continue
+        print("CASE", n, method, BC, flush=True)
+        got = []
+        for kind in (None, 0):
+            sol = hip.Solver((n,), method, 3, BC, -1.0, 0.9, 0.04, 0.004)
+            if kind is not None:
+                sol.set_kernel(kind, 8)
+            sol.set_state(U, V)
+            sol.step(37)
+            sol.step(3)
+            got.append(sol.state())
+            sol.close()
+        assert bits_equal(*got), BC
