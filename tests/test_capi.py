@@ -84,3 +84,20 @@ def test_vorticity_argument_checks_need_no_gpu():
     assert rc == 1 and b"null solver" in L.nlse_last_error()
     with pytest.raises(ValueError):
         nm.rmc_vorticity3D(np.zeros((4, 4)), 0.5, 1e-3)
+
+
+@pytest.mark.parametrize("shape", [(401,), (131, 150), (48, 50, 52)])
+@pytest.mark.parametrize("method", [1, 2])
+@pytest.mark.parametrize("precision", [1, 2, 3])
+def test_footprint_is_what_create_allocates(shape, method, precision):
+    """U, Y0, Y1, ktot with the staging pad, V, D in 3D 2SHOC, the low part of a
+    compensated state, and the reduction workspace."""
+    import nlsemagic_amd as nm
+    n = 1
+    for s in shape:
+        n *= s
+    e = 16 if precision == 2 else 8
+    ext = sum(shape) + (3 - len(shape))
+    expect = 4 * n * e + 16 + n * e // 2 + 8 * (6 * 1024 + 16 + 4 * ext)
+    expect += n * e * ((len(shape) == 3 and method == 2) + (precision == 3))
+    assert nm.footprint_bytes(shape, method, precision) == expect
