@@ -1,6 +1,7 @@
 // nlse2d_batch.hip -- many independent 2D problems (uneven sizes, own s, a,
 // h, k and V each) advanced by ONE launch per fused group of RK4
-// stages.  Each workgroup walks the concatenated tile list of all problems;
+// stages, over the concatenated tile list of all problems: by default a
+// workgroup per tile for row-sweep tiles, fewer that walk the list otherwise;
 // the tile code is the single-problem one (nlse2d_tile.h, nlse2d_rows.h,
 // nlse2d_strip.h), so every problem's result is bit-identical to running it
 // alone.
@@ -10,7 +11,7 @@
 
 namespace nlse {
 
-// The grid walks the concatenated tile list of all problems: block b
+// A grid of workgroups walks the concatenated tile list of all problems: block b
 // works on XCD b mod 8, which owns a contiguous eighth of the list, so the
 // tiles of one problem (and their shared halos) stay in one L2.
 template <typename T, int METHOD, int TI, int FIRST, int LAST>

@@ -1,6 +1,6 @@
 // nlse2d_rows.h -- row-sweep LDS tile for fused 2D RK4 stages (device code).
 //
-// A workgroup of NW (4 or 8) waves advances a tile of TI rows x W = 64 - 2H owned
+// A workgroup of NW (4, 8 or 16) waves advances a tile of TI rows x W = 64 - 2H owned
 // columns through RK4 stages FIRST..LAST (H = R per fused stage):
 //   - lane l is column j0 - H + l, so one row of the extended tile (the owned
 //     block plus H rows/columns of halo) is exactly one wave-wide access:
@@ -20,9 +20,9 @@
 //     lane shifts FP64 15.8 -> 16.3 us, FP32 equal);
 //   - per stage: D phase, barrier, F phase (each row's F and RK4 update at
 //     once, the new Y in the row's registers), barrier, new Y rows written
-//     to LDS, barrier (rows_early(): the corner terms in the D phase, the new Y
-//     to LDS in the F phase, one barrier less); the last stage writes its rows
-//     to HBM.
+//     to LDS, barrier (rows_early(), tiles without row 0 or N-1: the corner terms
+//     in the D phase, the new Y to LDS in the F phase, one barrier less); the last
+//     stage writes its rows to HBM.
 // MSD boundary rows take their partner row's D/F from LDS after the barrier
 // that completes it (D: one extra barrier, only in tiles holding row 0 or
 // N-1).  MSD boundary columns take the partner lane's F by DPP; their D is
@@ -176,7 +176,7 @@ __device__ __forceinline__ void rows2d_tile(RowsLds<T, METHOD, FIRST, LAST, TI>&
 
     constexpr bool EARLY = RIN && rows_early<T, METHOD, FIRST, LAST, NW>();
 
-    // rows of this wave: e = 4k + w; everything about row e stays in slot k
+    // rows of this wave: e = NW k + w; everything about row e stays in slot k
     c2<T> Yc[RW], Uc[RW], Ac[RW], Lc[RW];
     T Vc[RW];
 

@@ -32,7 +32,7 @@
 // and at 256^3 the loads (1.75 us per plane).  Before, one row per wave on 12
 // waves and 4 owned rows (FP64) kept four planes of every array in LDS: about
 // 1760 clocks of LDS reads and writes per plane for half the rows.  Per RK4
-// step at 256^3 (chunks as now): FP64 1014 -> 702 us, FP32c 548 -> 433 us;
+// step at 256^3 (chunks as now): FP64 1014 -> 705 us, FP32c 548 -> 433 us;
 // 128^3 FP64 194 -> 121 us.  12 waves (TJ = 8, FP64) leave 168 VGPRs, 16
 // (TJ = 12, FP32) 128; TJ = 4 in FP64 and 8 in FP32 were slower at every size
 // of 96^3 and more (256^3: 926 and 471 us).

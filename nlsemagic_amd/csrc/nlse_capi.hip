@@ -389,7 +389,7 @@ template <typename S> hipError_t get_kernel(const StateRef& h, Pieces<S> dst)
     return hipGetLastError();
 }
 
-// States of up to this many bytes of host arrays go through one pinned block
+// States of up to this many bytes go through one pinned block
 // that the conversion kernel reads or writes over PCIe: a launch and a host
 // copy in place of two or three DMA copies with their own submissions.  FP64
 // upload of U and V / download: 2048 points 31 / 23 -> 17 / 14 us, 32768

@@ -31,11 +31,16 @@
 //
 // Rows and planes inside the grid, in tiles without column 0 or M-1, run
 // central differences only (uniform branch); the others select operands per
-// lane, without branches.  Bound: HBM at 256^3 (the 48 B a point needs take
-// 159 us at the rate of a large copy).  Per call, 16 rows on 16 waves with a
-// branch per difference and loads widened at once -> this: 256^3 FP64 244 ->
-// 151 us, FP32 275 -> 149, FP32c 333 -> 158; 201 x 180 x 190 FP64 150 -> 99;
-// 64^3 FP64 68 -> 14; 256^3 of four vortex rings 258 -> 191.
+// lane, without branches.  At 256^3 the bytes a point needs take 159 us at the
+// rate of a large copy (48 B: FP64, FP32 compensated) or 133 us (FP32, 40 B).  A
+// call takes about the same in every precision: the four outputs and the plane
+// step's chain of loads, differences and division bound it, not the state's
+// bytes, of which repeated calls find a part in the 256 MB cache.  The time
+// depends on the values (clock): a uniform state FP64 151 us, FP32 149, FP32c 158,
+// four vortex rings 173, 163 and 179.  Per call, 16 rows on 16 waves with a branch
+// per difference and loads widened at once -> this: uniform 256^3 FP64 244 -> 151
+// us, FP32 275 -> 149, FP32c 333 -> 158; 201 x 180 x 190 FP64 150 -> 99; 64^3 FP64
+// 68 -> 14; four rings of 256^3 in a run of 20 calls 258 -> 191.
 #include "nlse2d_strip.h"
 #include "nlse_host.h"
 
