@@ -1498,7 +1498,8 @@ int nlse_get_config(const nlse_solver* h, int* fusion_out, int* kind, int* rows)
 int nlse_autotune(nlse_solver* h, int steps, int* best_fusion, int* best_tile, double* best_ms)
 {
     if (!h || steps <= 0) return fail(NLSE_EINVAL, "bad argument");
-    if (h->dim == 1 || (h->dim == 3 && h->BC == BC_MSD)) {  // nothing to tune; report what is in use
+    // 1D has nothing to tune, 3D MSD keeps its rule (msd_pairs): report what is in use
+    if (h->dim == 1 || (h->dim == 3 && h->BC == BC_MSD)) {
         if (best_fusion) *best_fusion = fusion(h);
         if (best_tile) *best_tile = 0;
         if (best_ms) *best_ms = 0;
